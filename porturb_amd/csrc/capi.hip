@@ -60,7 +60,7 @@ template <class P> static int alloc(P **p, size_t bytes) {
 }
 
 static void free_ctx(pu_ctx *c) {
-  void *ptrs[] = {c->d_hy, c->d_imm_flag, c->d_any10, c->d_tau, c->d_relax, c->d_imm_les, c->d_imm_les_val,
+  void *ptrs[] = {c->d_hy, c->d_codes, c->d_any10, c->d_tau, c->d_relax, c->d_imm_les, c->d_imm_les_val,
                   c->d_U, c->d_Us, c->d_Ulo, c->d_Uslo, c->d_tend, c->d_prim, c->d_les, c->d_red,
                   c->d_sgs_tau, c->d_sgs_flags, c->d_sgs_valid, c->d_sgs_fmul, c->d_sfc_rough, c->d_sfc_temp,
                   c->d_col};
@@ -111,7 +111,7 @@ int pu_create(const pu_config *cfg, void *stream, pu_ctx **out) {
   int nq = 0;
   for (int tr = 0; tr < cfg->num_tracers; tr++) nq += cfg->tracer_diffuse[tr] ? 1 : 0;
   if ((rc = alloc(&c->d_hy, sizeof(double) * (3 * (g.nz + 2 * g.hs) + 3 * (g.nz + 1)))) ||
-      (rc = alloc(&c->d_imm_flag, nh)) || (rc = alloc(&c->d_any10, n3)) || (rc = alloc(&c->d_tau, n3 * sizeof(int))) ||
+      (rc = alloc(&c->d_codes, 3 * n3 * sizeof(uint16_t))) || (rc = alloc(&c->d_any10, n3)) || (rc = alloc(&c->d_tau, n3 * sizeof(int))) ||
       (rc = alloc(&c->d_relax, n3 * sizeof(double))) || (rc = alloc(&c->d_imm_les_val, nl * sizeof(double))) || (rc = alloc(&c->d_imm_les, nl)) ||
       (rc = alloc(&c->d_U, es * c->nv * n3)) || (rc = alloc(&c->d_Us, es * c->nv * n3)) ||
       (rc = alloc(&c->d_tend, es * c->nv * n3)) || (rc = alloc(&c->d_prim, es * c->nf * nh)) ||

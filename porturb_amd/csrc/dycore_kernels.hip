@@ -259,28 +259,33 @@ __global__ __launch_bounds__(256) void k_tend_export(const ST *__restrict__ tend
 // given state.  grid: (blocks over a level's nx*ny cells, nz levels).
 // ------------------------------------------------------------------------------------------------
 template <int ORD, class T, int DIR>
-__global__ __launch_bounds__(256) void k_flat_census(const T *__restrict__ prim, const uint8_t *__restrict__ immf,
-                                                     const uint8_t *__restrict__ any10, SweepParams P,
-                                                     unsigned long long *counts) {
+__global__ __launch_bounds__(256) void k_flat_census(const T *__restrict__ prim, const uint16_t *__restrict__ codes,
+                                                     SweepParams P, unsigned long long *counts) {
   __shared__ unsigned long long sc[3];
   if (threadIdx.x < 3) sc[threadIdx.x] = 0;
   __syncthreads();
+  constexpr int hs = (ORD - 1) / 2;
   const int nxy = P.nx * P.ny;
   const int p = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
   unsigned c[3] = {0u, 0u, 0u};
   if (p < nxy) {
     const int i = p % P.nx, j = p / P.nx;
     const long long sstride = DIR == 0 ? 1 : (DIR == 1 ? P.nxh : P.nxh * P.nyh);
-    const long long base = ((long long)(k + P.hp) * P.nyh + (j + P.hp)) * P.nxh + (i + P.ox);
-    const long long cid = (long long)k * nxy + p;
-    StencilFlags<ORD> sf;
-    sf.setup(immf, base, sstride, any10[cid] != 0, P.weno_all);
+    const long long base = ((long long)(k + P.hp) * P.nyh + (j + P.hp)) * P.nxh + (i + P.ox) - hs * sstride;
+    const unsigned code = codes[(long long)k * nxy + p];
+    const bool weno = P.weno_all || (code & SC_ANY);
+    // the branch the sweeps take: 0 the limiter, 1 flat stencil, 2 a cell without WENO
+    auto branch = [&](int l, bool clamp) {
+      if (!weno) return 2;
+      T s[ORD], dif[ORD - 1], TV[pu_weno::Ops<ORD>::S];
+      load_stencil<ORD, T, long long>(prim + (long long)l * P.nh, sstride, base * (long long)sizeof(T), code, clamp, s);
+      return flat_stencil(variations<ORD, T>(s, dif, TV)) ? 1 : 0;
+    };
     constexpr int ln = 1 + DIR, lt1 = DIR == 0 ? idV : idU, lt2 = DIR == 2 ? idV : idW;
     const int ls[5] = {idR, ln, idP, lt1, lt2};
-    for (int f = 0; f < 5; f++) c[sf.template branch<T>(prim + (long long)ls[f] * P.nh + base, sstride, f >= 2)]++;
-    c[sf.template branch<T>(prim + (long long)idT * P.nh + base, sstride, false)]++;
-    for (int tr = 0; tr < P.ntr; tr++)
-      c[sf.template branch<T>(prim + (long long)(NUM_STATE + 1 + tr) * P.nh + base, sstride, false)]++;
+    for (int f = 0; f < 5; f++) c[branch(ls[f], f >= 2)]++;
+    c[branch(idT, false)]++;
+    for (int tr = 0; tr < P.ntr; tr++) c[branch(NUM_STATE + 1 + tr, false)]++;
   }
   for (int q = 0; q < 3; q++) if (c[q]) atomicAdd(&sc[q], (unsigned long long)c[q]);
   __syncthreads();
@@ -333,69 +338,73 @@ static SweepParams sweep_params(pu_ctx *ctx, int dir) {
   return P;
 }
 
-// mode: 0 first sweep (writes d_tend), 1 adds to d_tend, 2 adds and combines stage `stage`
-template <int ORD, class T, int DIR>
-static int sweep_one(pu_ctx *ctx, hipStream_t s, int mode, int stage, double dt, int nrelax) {
+// z sweep: writes d_tend.  Between solid walls the whole-column kernel, otherwise (periodic z, or
+// columns whose offsets need more than 32 bits) the segment kernel.
+template <int ORD, class T>
+static int sweep_z(pu_ctx *ctx, hipStream_t s) {
   const pu::Grid &g = ctx->g;
-  SweepParams P = sweep_params(ctx, DIR);
-  static const char *names[3] = {"weno_x", "weno_y", "weno_z"};
-  LaunchTimer lt(ctx, names[DIR]);
-  constexpr int BX = SegShape<DIR>::BX, BY = SegShape<DIR>::BY, NC = SegShape<DIR>::BS - 2;
-  dim3 blk(BX, BY, 1), grd;
-  if (DIR == 0) grd = dim3((unsigned)((g.nx + NC - 1) / NC), (unsigned)((g.ny + BY - 1) / BY), (unsigned)g.nz);
-  else if (DIR == 1) grd = dim3((unsigned)((g.nx + BX - 1) / BX), (unsigned)((g.ny + NC - 1) / NC), (unsigned)g.nz);
-  else grd = dim3((unsigned)((g.nx + BX - 1) / BX), (unsigned)g.ny, (unsigned)((g.nz + NC - 1) / NC));
-  FuseArgs<T> FA{};
+  SweepParams P = sweep_params(ctx, 2);
+  LaunchTimer lt(ctx, "weno_z");
   const T *prim = (const T *)ctx->d_prim;
   T *tend = (T *)ctx->d_tend;
-  constexpr bool line_kernel =
-      DIR <= 1 && ((PU_PLINE >> ((DIR == 0 ? 1 : 0) + (std::is_same<T, float>::value ? 2 : 0))) & 1);
-  if constexpr (line_kernel) {
-    if (!ctx->segment_sweeps[DIR] && mode >= 1 && P.bc_along == PU_BC_PERIODIC && (DIR == 0 ? g.nx : g.ny) >= 2) {
-      constexpr int D = DIR <= 1 ? DIR : 0;
-      dim3 lb(LineShape<D>::BX, LineShape<D>::BY, 1);
-      dim3 lg(DIR == 0 ? (unsigned)((g.ny + lb.y - 1) / lb.y) : (unsigned)((g.nx + lb.x - 1) / lb.x), (unsigned)g.nz, 1);
-      if constexpr (std::is_same<T, float>::value && DIR == 1) {
-        // FP32 y lines: their own translation unit (sweep_pline_f32.hip); y never combines the stage
-        if (mode != 1) return fail(PU_ERR_ARG, "the y sweep does not combine the stage");
-        const int rc = launch_pline_y_f32(ORD, lg, lb, s, prim, ctx->d_imm_flag, ctx->d_any10, tend, P, FA);
-        if (rc) return rc;
-      } else if (mode == 2) {
-        FA.U = (T *)ctx->d_U; FA.Ulo = (T *)ctx->d_Ulo; FA.Us = (T *)ctx->d_Us; FA.Uslo = (T *)ctx->d_Uslo;
-        FA.C = combine_params(ctx);
-        FA.C.stage = stage; FA.C.dt = dt; FA.C.nrelax = nrelax;
-        hipLaunchKernelGGL((k_sweep_pline<ORD, T, D, 2>), lg, lb, 0, s, prim, ctx->d_imm_flag, ctx->d_any10, tend, P, FA);
-      } else {
-        hipLaunchKernelGGL((k_sweep_pline<ORD, T, D, 1>), lg, lb, 0, s, prim, ctx->d_imm_flag, ctx->d_any10, tend, P, FA);
-      }
-      PU_HIP_CHECK(hipGetLastError());
-      return PU_OK;
-    }
+  const uint16_t *codes = ctx->d_codes + 2 * g.n3();
+  if (!ctx->segment_sweeps[2] && P.wall_z && offsets_fit<T>(g.nxh * g.nyh, g.hp)) {
+    const dim3 blk(ZW_BX, ZW_BS, 1), grd((unsigned)((g.nx + ZW_BX - 1) / ZW_BX), (unsigned)g.ny, 1);
+    if constexpr (std::is_same<T, float>::value) return launch_zwall_f32(ORD, grd, blk, s, prim, codes, tend, P);
+    else hipLaunchKernelGGL((k_sweep_zwall<ORD, T>), grd, blk, 0, s, prim, codes, tend, P);
+  } else {
+    const dim3 blk(SG_BX, SG_BS, 1);
+    const dim3 grd((unsigned)((g.nx + SG_BX - 1) / SG_BX), (unsigned)g.ny, (unsigned)((g.nz + SG_NC - 1) / SG_NC));
+    hipLaunchKernelGGL((k_sweep_seg<ORD, T, 2>), grd, blk, 0, s, prim, codes, tend, P);
   }
-  if (PU_ZWALL && !ctx->segment_sweeps[2] && DIR == 2 && mode == 0 && ctx->cfg.bc_z == PU_BC_SOLID_WALL) {
-    dim3 zb(ZW_BX, ZW_BS, 1), zg((unsigned)((g.nx + ZW_BX - 1) / ZW_BX), (unsigned)g.ny, 1);
-    if constexpr (std::is_same<T, float>::value) {
-      const int rc = launch_zwall_f32(ORD, zg, zb, s, prim, ctx->d_imm_flag, ctx->d_any10, tend, P);
-      if (rc) return rc;
-    } else {
-      hipLaunchKernelGGL((k_sweep_zwall<ORD, T>), zg, zb, 0, s, prim, ctx->d_imm_flag, ctx->d_any10, tend, P);
-    }
-  } else if (mode == 2) {
+  PU_HIP_CHECK(hipGetLastError());
+  return PU_OK;
+}
+
+// y sweep: adds to d_tend.  Periodic lines the whole-line kernel, otherwise the segment kernel.
+template <int ORD, class T>
+static int sweep_y(pu_ctx *ctx, hipStream_t s) {
+  const pu::Grid &g = ctx->g;
+  SweepParams P = sweep_params(ctx, 1);
+  LaunchTimer lt(ctx, "weno_y");
+  const T *prim = (const T *)ctx->d_prim;
+  T *tend = (T *)ctx->d_tend;
+  const uint16_t *codes = ctx->d_codes + g.n3();
+  if (!ctx->segment_sweeps[1] && P.bc_along == PU_BC_PERIODIC && offsets_fit<T>(g.nxh, g.hp)) {
+    const dim3 blk(YL_BX, YL_BS, 1), grd((unsigned)((g.nx + YL_BX - 1) / YL_BX), (unsigned)g.nz, 1);
+    if constexpr (std::is_same<T, float>::value) return launch_yline_f32(ORD, grd, blk, s, prim, codes, tend, P);
+    else hipLaunchKernelGGL((k_sweep_yline<ORD, T>), grd, blk, 0, s, prim, codes, tend, P);
+  } else {
+    const dim3 blk(SG_BX, SG_BS, 1);
+    const dim3 grd((unsigned)((g.nx + SG_BX - 1) / SG_BX), (unsigned)((g.ny + SG_NC - 1) / SG_NC), (unsigned)g.nz);
+    hipLaunchKernelGGL((k_sweep_seg<ORD, T, 1>), grd, blk, 0, s, prim, codes, tend, P);
+  }
+  PU_HIP_CHECK(hipGetLastError());
+  return PU_OK;
+}
+
+// x sweep: adds to d_tend (stage < 0) or finishes the tendencies and combines the stage
+template <int ORD, class T>
+static int sweep_x(pu_ctx *ctx, hipStream_t s, int stage, double dt, int nrelax) {
+  const pu::Grid &g = ctx->g;
+  SweepParams P = sweep_params(ctx, 0);
+  LaunchTimer lt(ctx, "weno_x");
+  const dim3 blk(SX_BX, SX_BY, 1);
+  const dim3 grd((unsigned)((g.nx + SX_NC - 1) / SX_NC), (unsigned)((g.ny + SX_BY - 1) / SX_BY), (unsigned)g.nz);
+  const T *prim = (const T *)ctx->d_prim;
+  T *tend = (T *)ctx->d_tend;
+  FuseArgs<T> FA{};
+  if (stage >= 0) {
     FA.U = (T *)ctx->d_U; FA.Ulo = (T *)ctx->d_Ulo; FA.Us = (T *)ctx->d_Us; FA.Uslo = (T *)ctx->d_Uslo;
     FA.C = combine_params(ctx);
     FA.C.stage = stage; FA.C.dt = dt; FA.C.nrelax = nrelax;
-    if constexpr (std::is_same<T, float>::value && DIR == 0)
-      return launch_seg_x_f32(ORD, 2, grd, blk, s, prim, ctx->d_imm_flag, ctx->d_any10, tend, P, FA);
-    else
-      hipLaunchKernelGGL((k_sweep<ORD, T, DIR, 2>), grd, blk, 0, s, prim, ctx->d_imm_flag, ctx->d_any10, tend, P, FA);
-  } else if constexpr (std::is_same<T, float>::value && DIR == 0) {
-    // FP32 x segments: their own translation unit (sweep_seg_x_f32.hip)
-    return launch_seg_x_f32(ORD, mode, grd, blk, s, prim, ctx->d_imm_flag, ctx->d_any10, tend, P, FA);
-  } else if (mode == 1) {
-    hipLaunchKernelGGL((k_sweep<ORD, T, DIR, 1>), grd, blk, 0, s, prim, ctx->d_imm_flag, ctx->d_any10, tend, P, FA);
-  } else {
-    hipLaunchKernelGGL((k_sweep<ORD, T, DIR, 0>), grd, blk, 0, s, prim, ctx->d_imm_flag, ctx->d_any10, tend, P, FA);
   }
+  if constexpr (std::is_same<T, float>::value)
+    return launch_x_f32(ORD, stage >= 0 ? 2 : 1, grd, blk, s, prim, ctx->d_codes, tend, P, FA);
+  else if (stage >= 0)
+    hipLaunchKernelGGL((k_sweep_x<ORD, T, 2>), grd, blk, 0, s, prim, ctx->d_codes, tend, P, FA);
+  else
+    hipLaunchKernelGGL((k_sweep_x<ORD, T, 1>), grd, blk, 0, s, prim, ctx->d_codes, tend, P, FA);
   PU_HIP_CHECK(hipGetLastError());
   return PU_OK;
 }
@@ -404,9 +413,9 @@ static int sweep_one(pu_ctx *ctx, hipStream_t s, int mode, int stage, double dt,
 template <int ORD, class T>
 static int sweeps_t(pu_ctx *ctx, hipStream_t s, int stage, double dt, int nrelax) {
   int rc;
-  if ((rc = sweep_one<ORD, T, 2>(ctx, s, 0, stage, dt, nrelax))) return rc;
-  if (ctx->g.ny > 1 && (rc = sweep_one<ORD, T, 1>(ctx, s, 1, stage, dt, nrelax))) return rc;
-  if ((rc = sweep_one<ORD, T, 0>(ctx, s, stage >= 0 ? 2 : 1, stage, dt, nrelax))) return rc;
+  if ((rc = sweep_z<ORD, T>(ctx, s))) return rc;
+  if (ctx->g.ny > 1 && (rc = sweep_y<ORD, T>(ctx, s))) return rc;
+  if ((rc = sweep_x<ORD, T>(ctx, s, stage, dt, nrelax))) return rc;
   return PU_OK;
 }
 
@@ -427,12 +436,12 @@ static int census_t(pu_ctx *ctx, hipStream_t s, unsigned long long *counts) {
   const pu::Grid &g = ctx->g;
   dim3 grd((unsigned)((g.nx * g.ny + 255) / 256), (unsigned)g.nz), blk(256);
   const T *prim = (const T *)ctx->d_prim;
-  hipLaunchKernelGGL((k_flat_census<ORD, T, 0>), grd, blk, 0, s, prim, ctx->d_imm_flag, ctx->d_any10,
+  hipLaunchKernelGGL((k_flat_census<ORD, T, 0>), grd, blk, 0, s, prim, ctx->d_codes,
                      sweep_params(ctx, 0), counts);
   if (g.ny > 1)
-    hipLaunchKernelGGL((k_flat_census<ORD, T, 1>), grd, blk, 0, s, prim, ctx->d_imm_flag, ctx->d_any10,
+    hipLaunchKernelGGL((k_flat_census<ORD, T, 1>), grd, blk, 0, s, prim, ctx->d_codes + g.n3(),
                        sweep_params(ctx, 1), counts + 3);
-  hipLaunchKernelGGL((k_flat_census<ORD, T, 2>), grd, blk, 0, s, prim, ctx->d_imm_flag, ctx->d_any10,
+  hipLaunchKernelGGL((k_flat_census<ORD, T, 2>), grd, blk, 0, s, prim, ctx->d_codes + 2 * g.n3(),
                      sweep_params(ctx, 2), counts + 6);
   PU_HIP_CHECK(hipGetLastError());
   return PU_OK;

@@ -209,17 +209,31 @@ def tv_ldl(ord_):
     return out
 
 
-def _lin_expr(coefs, var):
+def _diff_expr(coefs, var):
     """Straight-line sum of the nonzero terms c*var[i] (left to right)."""
     terms = ["T(%s)*%s[%d]" % (lit(c), var, i) for i, c in enumerate(coefs) if c != 0]
     return " + ".join(terms) if terms else "T(0)"
 
 
+def face_differences(ord_, side):
+    """Each candidate's face value minus the cell's own average as weights over the first
+    differences d_j = s_{j+1} - s_j (a candidate's face weights sum to one and its points include
+    the cell, so the difference is a combination of its d_j): weight of d_j is the sum of the face
+    weights of the points above it for j >= hs, minus that of the points up to it for j < hs."""
+    t = tables(ord_)
+    hs = t["hs"]
+    out = []
+    for row in t["face"][side]:
+        out.append([sum(row[j + 1:]) if j >= hs else -sum(row[:j + 1]) for j in range(ord_ - 1)])
+    return out
+
+
 def emit_ops(path):
-    """Device code: one struct per order with the TV, face and linear expressions written out."""
+    """Device code: one struct per order with the TV and face expressions written out."""
     out = []
     out.append("// Generated by gen_weno_tables.py -- WENO reconstruction expressions (device code).")
     out.append("// Do not edit by hand.  Only nonzero coefficients appear.")
+    out.append("// d: first differences of the stencil, d[i] = s[i + 1] - s[i].")
     out.append("#pragma once")
     out.append("#include <hip/hip_runtime.h>")
     out.append("namespace pu_weno {")
@@ -231,10 +245,7 @@ def emit_ops(path):
         out.append("  static constexpr int ord = %d, hs = %d, N = %d, S = %d;" % (ord_, hs, N, S))
         out.append("  static constexpr bool use_map_rs = %s;" % ("true" if ord_ > 3 else "false"))
         # TV of each sub-stencil: sum of D_k * (first-difference combination)^2 (see tv_ldl)
-        out.append("  template <class T> __device__ static __forceinline__ void tv(const T *s, T *TV) {")
-        out.append("    T d[%d];" % (ord_ - 1))
-        out.append("    #pragma unroll")
-        out.append("    for (int i = 0; i < %d; i++) d[i] = s[i + 1] - s[i];" % (ord_ - 1))
+        out.append("  template <class T> __device__ static __forceinline__ void tv(const T *d, T *TV) {")
         for m, (Dk, L) in enumerate(tv_ldl(ord_)):
             n = N - 1
             terms = []
@@ -248,16 +259,12 @@ def emit_ops(path):
             out.append("    TV[%d] = %s;" % (m, " + ".join(terms)))
         out.append("  }")
         for side in ("L", "R"):
-            out.append("  template <class T> __device__ static __forceinline__ T comb%s(const T *s, const T *w) {" % side)
-            parts = []
-            for m in range(S):
-                parts.append("(%s)*w[%d]" % (_lin_expr(t["face"][side][m], "s"), m))
-            out.append("    return %s;" % " + ".join(parts))
+            # e[m]: candidate m's value at the face minus the cell average
+            out.append("  template <class T> __device__ static __forceinline__ void edge%s(const T *d, T *e) {" % side)
+            for m, row in enumerate(face_differences(ord_, side)):
+                out.append("    e[%d] = %s;" % (m, _diff_expr(row, "d")))
             out.append("  }")
-            out.append("  template <class T> __device__ static __forceinline__ T lin%s(const T *s) {" % side)
-            out.append("    return %s;" % _lin_expr(t["lin"][side], "s"))
-            out.append("  }")
-            out.append("  __device__ static __forceinline__ double ideal%s(int m) {" % side)
+            out.append("  __device__ static __forceinline__ constexpr double ideal%s(int m) {" % side)
             out.append("    constexpr double d[%d] = {%s};" % (S, ",".join(lit(v) for v in t["ideal"][side])))
             out.append("    return d[m];")
             out.append("  }")

@@ -103,6 +103,30 @@ __global__ __launch_bounds__(256) void k_imm_flag(const double *prop, uint8_t *f
   flag[id] = v > 0 ? 1 : 0;
 }
 
+// Stencil codes of the sweeps along x, y and z (dynamics_rk.h:572-607 with
+// modify_stencil_immersed_der0, :478-493), fixed once the immersed cells are: how many points at
+// either end of a cell's stencil lie behind an immersed cell (0 for an immersed cell itself),
+// whether its two neighbours are immersed, and whether its 10-cell box holds an immersed cell.  The
+// sweeps read 2 bytes per cell instead of deriving them from 2 hs + 2 flag bytes in every launch.
+__global__ __launch_bounds__(256) void k_stencil_codes(const uint8_t *flag, const uint8_t *any10, uint16_t *codes,
+                                                       ImmParams P) {
+  const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (id >= P.n3) return;
+  const int i = (int)(id % P.nx), j = (int)((id / P.nx) % P.ny), k = (int)(id / ((long long)P.nx * P.ny));
+  const uint8_t *f = flag + ((long long)(k + P.hp) * P.nyh + (j + P.hp)) * P.nxh + (i + P.ox);
+  for (int d = 0; d < 3; d++) {
+    const long long st = d == 0 ? 1 : (d == 1 ? P.nxh : P.nxh * P.nyh);
+    int lo = 0, gap = 0;
+    if (!f[0]) {
+      for (int s = P.hs; s >= 1; s--) {          // the nearest immersed point decides
+        if (f[-s * st]) lo = P.hs - s + 1;
+        if (f[s * st]) gap = P.hs - s + 1;
+      }
+    }
+    codes[d * P.n3 + id] = (uint16_t)(lo | (gap << 4) | (f[-st] ? 0x100 : 0) | (f[st] ? 0x200 : 0) | (any10[id] ? 0x400 : 0));
+  }
+}
+
 // immersed tau (dynamics_rk.h:389-425) and relaxation multiplier pow(prop, power)/tau (:429)
 __global__ __launch_bounds__(256) void k_tau_relax(const double *prop, int *tau, double *relax, ImmParams P) {
   long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -290,18 +314,18 @@ static int build_immersed(pu_ctx *ctx, const double *prop) {
   ImmParams P;
   P.nx = g.nx; P.ny = g.ny; P.nz = g.nz; P.hs = g.hs; P.hp = g.hp; P.ox = g.ox;
   P.nxh = g.nxh; P.nyh = g.nyh; P.nzh = g.nzh; P.n3 = n3; P.power = c.immersed_power;
-  long long nh = g.nh();
-  hipLaunchKernelGGL(k_imm_flag, dim3((unsigned)((nh + 255) / 256)), dim3(256), 0, s, prop, ctx->d_imm_flag, P);
-  PU_HIP_CHECK(hipGetLastError());
   dim3 grd((unsigned)((n3 + 255) / 256)), blk(256);
   hipLaunchKernelGGL(k_tau_relax, grd, blk, 0, s, prop, ctx->d_tau, ctx->d_relax, P);
   PU_HIP_CHECK(hipGetLastError());
-  uint8_t *tmp1 = nullptr, *tmp2 = nullptr;
-  PU_HIP_CHECK(hipMalloc(&tmp1, n3));
+  const long long nh = g.nh();
+  uint8_t *tmp1 = nullptr, *tmp2 = nullptr;      // tmp1: a filter's result, then the halo'd flags
+  PU_HIP_CHECK(hipMalloc(&tmp1, nh));
   PU_HIP_CHECK(hipMalloc(&tmp2, n3));
   hipLaunchKernelGGL(k_any_x, grd, blk, 0, s, prop, tmp1, P, 10);
   hipLaunchKernelGGL(k_any_y, grd, blk, 0, s, tmp1, tmp2, P, 10);
   hipLaunchKernelGGL(k_any_z, grd, blk, 0, s, tmp2, ctx->d_any10, P, 10);
+  hipLaunchKernelGGL(k_imm_flag, dim3((unsigned)((nh + 255) / 256)), blk, 0, s, prop, tmp1, P);
+  hipLaunchKernelGGL(k_stencil_codes, grd, blk, 0, s, tmp1, ctx->d_any10, ctx->d_codes, P);
   PU_HIP_CHECK(hipGetLastError());
   long long nl = (long long)(g.nx + 2) * (g.ny + 2) * (g.nz + 2);
   hipLaunchKernelGGL(k_imm_les, dim3((unsigned)((nl + 255) / 256)), blk, 0, s, prop, ctx->d_imm_les_val,

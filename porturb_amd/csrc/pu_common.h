@@ -60,7 +60,7 @@ struct pu_ctx {
   std::vector<double> hy_edges[3];     // [nz+1]
   double *d_hy = nullptr;              // device: [3*(nz+2hs)] cells then [3*(nz+1)] edges
   // immersed data
-  uint8_t *d_imm_flag = nullptr;       // (prop_halos > 0), halo'd with the primitive halo
+  uint16_t *d_codes = nullptr;         // stencil codes along x, y, z [3][n3] (sweep_core.h SC_*)
   uint8_t *d_any10 = nullptr;          // dycore_any_immersed10 [n3]
   int     *d_tau = nullptr;            // dycore_immersed_tau [n3]
   double  *d_relax = nullptr;          // pow(prop, immersed_power)/tau [n3]

@@ -14,8 +14,8 @@ import gen_weno_tables as _gen  # noqa: E402
 MI355X = {"hbm_GBps": 8000.0, "fp64_TFLOPs": 78.6, "fp32_TFLOPs": 157.3}
 
 
-def recon_flops(ord_, do_map=True):
-    """Both interface values of one field in one cell (weno_edges, WENO branch)."""
+def recon_flops(ord_, do_map=True, sides="LR"):
+    """Interface values of one field in one cell (WENO branch): both, or with sides="R" one."""
     t = _gen.tables(ord_)
     N, S = t["N"], t["S"]
     f = 0
@@ -29,12 +29,12 @@ def recon_flops(ord_, do_map=True):
     conv = (S - 1) + 1 + S
     f += conv                       # normalise TV
     f += 3 * S                      # 1/(TV^2 + eps)
-    f += 2 * S                      # ideal * 1/(...)
-    f += 2 * conv
+    f += len(sides) * S             # ideal * 1/(...)
+    f += len(sides) * conv
     if do_map:
-        f += 2 * S * (14 if ord_ > 3 else 9)
-        f += 2 * conv
-    for side in ("L", "R"):
+        f += len(sides) * S * (14 if ord_ > 3 else 9)
+        f += len(sides) * conv
+    for side in sides:
         for m in range(S):
             nnz = sum(1 for v in t["face"][side][m] if v != 0)
             f += 2 * nnz - 1
@@ -57,16 +57,22 @@ def _tv_flops(ord_):
     return f + (S - 1)
 
 
-def linear_flops(ord_):
-    """Both interface values from the full-stencil polynomial (the linear reconstruction)."""
+def linear_flops(ord_, sides="LR"):
+    """Interface values from the full-stencil polynomial (the linear reconstruction)."""
     t = _gen.tables(ord_)
-    return sum(2 * sum(1 for v in t["lin"][side] if v != 0) - 1 for side in ("L", "R"))
+    return sum(2 * sum(1 for v in t["lin"][side] if v != 0) - 1 for side in sides)
 
 
-def recon_flops_flat(ord_):
-    """Both interface values of a flat stencil (total variation <= 1e-20): the total variations
-    that decide the branch, then the linear reconstruction."""
-    return _tv_flops(ord_) + linear_flops(ord_)
+def recon_flops_flat(ord_, sides="LR"):
+    """Interface values of a flat stencil (total variation <= 1e-20): the total variations that
+    decide the branch, then the linear reconstruction."""
+    return _tv_flops(ord_) + linear_flops(ord_, sides)
+
+
+def per_field(nf, flops):
+    """Average over a sweep's nf fields of flops(sides): density, normal velocity and pressure are
+    reconstructed on both sides of a cell, the transported quantities on a face's upwind side."""
+    return (3 * flops("LR") + (nf - 3) * flops("R")) / nf
 
 
 def sweep_overhead_flops(nf):
@@ -80,16 +86,19 @@ def sweep_overhead_flops(nf):
 
 def executed_sweep_flops(ord_, nf, census_row, cells):
     """FLOPs one sweep launch executes over `cells` cells, from the reconstruction census of the
-    state (counts of the limiter, flat-stencil and linear branches)."""
+    state (counts of the limiter, flat-stencil and linear branches over all fields, so each branch
+    is priced at its average over the fields)."""
     n_lim, n_flat, n_lin = (int(v) for v in census_row)
-    return (n_lim * recon_flops(ord_) + n_flat * recon_flops_flat(ord_) + n_lin * linear_flops(ord_)
-            + cells * sweep_overhead_flops(nf))
+    return (n_lim * per_field(nf, lambda sides: recon_flops(ord_, sides=sides))
+            + n_flat * per_field(nf, lambda sides: recon_flops_flat(ord_, sides))
+            + n_lin * per_field(nf, lambda sides: linear_flops(ord_, sides)) + cells * sweep_overhead_flops(nf))
 
 
 def sweep_flops_per_cell(ord_, nf):
-    """One direction: nf reconstructions, the acoustic Riemann solve at one face, upwinded fluxes
-    and the flux divergence of nf-1 conserved variables."""
-    return nf * recon_flops(ord_) + sweep_overhead_flops(nf)
+    """One direction: nf reconstructions (three on both sides, the others on the upwind side), the
+    acoustic Riemann solve at one face, upwinded fluxes and the flux divergence of nf-1 conserved
+    variables."""
+    return nf * per_field(nf, lambda sides: recon_flops(ord_, sides=sides)) + sweep_overhead_flops(nf)
 
 
 def step_flops_per_cell(ord_, nf):
