@@ -96,17 +96,21 @@ def cpu_baseline(cfg_full, les, seconds_budget=25.0):
 
 def sweep_kernel_name(cfg, fam):
     """The kernel that runs sweep family `fam` (the launch choice of dycore_kernels.hip): z between
-    solid walls -> k_sweep_zwall, periodic y lines -> k_sweep_yline, x -> k_sweep_x (which finishes
-    the stage: MODE 2), otherwise the segment kernel k_sweep_seg<ORD, T, DIR>."""
+    solid walls and periodic y lines the line kernels, x k_sweep_x in FP64 (which finishes the
+    stage: MODE 2), otherwise the segment kernels (FP32 kernels live in namespace f32)."""
     import porturb_amd as pa
-    t = "double" if cfg["precision"] == pa.PU_FP64 else "float"
+    fp64 = cfg["precision"] == pa.PU_FP64
+    t, ns = ("double", "") if fp64 else ("float", "f32::")
     if fam == "weno_z" and cfg["bc_z"] == pa.PU_BC_SOLID_WALL:
-        return "k_sweep_zwall<%d, %s>" % (cfg["ord"], t)
+        return "%sk_sweep_zwall<%d, %s>" % (ns, cfg["ord"], t)
     if fam == "weno_y" and cfg["bc_y"] == pa.PU_BC_PERIODIC and cfg["ny"] >= 2:
-        return "k_sweep_yline<%d, %s>" % (cfg["ord"], t)
-    if fam == "weno_x":
+        return "%sk_sweep_yline<%d, %s>" % (ns, cfg["ord"], t)
+    if fam == "weno_x" and fp64:
         return "k_sweep_x<%d, %s, 2>" % (cfg["ord"], t)
-    return "k_sweep_seg<%d, %s, %d>" % (cfg["ord"], t, {"weno_y": 1, "weno_z": 2}[fam])
+    d = {"weno_x": 0, "weno_y": 1, "weno_z": 2}[fam]
+    if fp64:
+        return "k_sweep_seg<%d, %s, %d>" % (cfg["ord"], t, d)
+    return "f32::k_sweep<%d, %s, %d, %d>" % (cfg["ord"], t, d, {0: 2, 1: 1, 2: 0}[d])
 
 
 def snapshot(d):
@@ -237,8 +241,8 @@ def main():
     fp64 = cfg["precision"] == pa.PU_FP64
     drow = {"weno_x": 0, "weno_y": 1, "weno_z": 2}[dom]
     census = (census0 + census1) / 2.0
-    flops_full = n3 * rl.sweep_flops_per_cell(cfg["ord"], nf)
-    flops_exec = rl.executed_sweep_flops(cfg["ord"], nf, census[drow], n3)
+    flops_full = n3 * rl.sweep_flops_per_cell(cfg["ord"], nf, fp64)
+    flops_exec = rl.executed_sweep_flops(cfg["ord"], nf, census[drow], n3, fp64)
     achieved = flops_exec / (avg_ms * 1e-3) / 1e12
     achieved_full = flops_full / (avg_ms * 1e-3) / 1e12
     peak = rl.MI355X["fp64_TFLOPs"] if fp64 else rl.MI355X["fp32_TFLOPs"]

@@ -349,9 +349,11 @@ static int sweep_z(pu_ctx *ctx, hipStream_t s) {
   T *tend = (T *)ctx->d_tend;
   const uint16_t *codes = ctx->d_codes + 2 * g.n3();
   if (!ctx->segment_sweeps[2] && P.wall_z && offsets_fit<T>(g.nxh * g.nyh, g.hp)) {
-    const dim3 blk(ZW_BX, ZW_BS, 1), grd((unsigned)((g.nx + ZW_BX - 1) / ZW_BX), (unsigned)g.ny, 1);
+    const dim3 blk(CH_BX, CH_BS, 1), grd((unsigned)((g.nx + CH_BX - 1) / CH_BX), (unsigned)g.ny, 1);
     if constexpr (std::is_same<T, float>::value) return launch_zwall_f32(ORD, grd, blk, s, prim, codes, tend, P);
     else hipLaunchKernelGGL((k_sweep_zwall<ORD, T>), grd, blk, 0, s, prim, codes, tend, P);
+  } else if constexpr (std::is_same<T, float>::value) {
+    return launch_seg_f32(ORD, 2, false, s, prim, codes, tend, P, FuseArgs<float>{});
   } else {
     const dim3 blk(SG_BX, SG_BS, 1);
     const dim3 grd((unsigned)((g.nx + SG_BX - 1) / SG_BX), (unsigned)g.ny, (unsigned)((g.nz + SG_NC - 1) / SG_NC));
@@ -371,9 +373,11 @@ static int sweep_y(pu_ctx *ctx, hipStream_t s) {
   T *tend = (T *)ctx->d_tend;
   const uint16_t *codes = ctx->d_codes + g.n3();
   if (!ctx->segment_sweeps[1] && P.bc_along == PU_BC_PERIODIC && offsets_fit<T>(g.nxh, g.hp)) {
-    const dim3 blk(YL_BX, YL_BS, 1), grd((unsigned)((g.nx + YL_BX - 1) / YL_BX), (unsigned)g.nz, 1);
+    const dim3 blk(CH_BX, CH_BS, 1), grd((unsigned)((g.nx + CH_BX - 1) / CH_BX), (unsigned)g.nz, 1);
     if constexpr (std::is_same<T, float>::value) return launch_yline_f32(ORD, grd, blk, s, prim, codes, tend, P);
     else hipLaunchKernelGGL((k_sweep_yline<ORD, T>), grd, blk, 0, s, prim, codes, tend, P);
+  } else if constexpr (std::is_same<T, float>::value) {
+    return launch_seg_f32(ORD, 1, false, s, prim, codes, tend, P, FuseArgs<float>{});
   } else {
     const dim3 blk(SG_BX, SG_BS, 1);
     const dim3 grd((unsigned)((g.nx + SG_BX - 1) / SG_BX), (unsigned)((g.ny + SG_NC - 1) / SG_NC), (unsigned)g.nz);
@@ -397,10 +401,14 @@ static int sweep_x(pu_ctx *ctx, hipStream_t s, int stage, double dt, int nrelax)
   if (stage >= 0) {
     FA.U = (T *)ctx->d_U; FA.Ulo = (T *)ctx->d_Ulo; FA.Us = (T *)ctx->d_Us; FA.Uslo = (T *)ctx->d_Uslo;
     FA.C = combine_params(ctx);
-    FA.C.stage = stage; FA.C.dt = dt; FA.C.nrelax = nrelax;
+    FA.C.stage = stage; FA.C.nrelax = nrelax;
+    // U + dt L(U); 3/4 U + 1/4 (Us + dt L(Us)); 1/3 U + 2/3 (Us + dt L(Us))
+    FA.C.cu = stage == 0 ? 1. : (stage == 1 ? 3. / 4. : 1. / 3.);
+    FA.C.cs = stage == 0 ? 0. : (stage == 1 ? 1. / 4. : 2. / 3.);
+    FA.C.ct = stage == 0 ? dt : FA.C.cs * dt;
   }
   if constexpr (std::is_same<T, float>::value)
-    return launch_x_f32(ORD, stage >= 0 ? 2 : 1, grd, blk, s, prim, ctx->d_codes, tend, P, FA);
+    return launch_seg_f32(ORD, 0, stage >= 0, s, prim, ctx->d_codes, tend, P, FA);
   else if (stage >= 0)
     hipLaunchKernelGGL((k_sweep_x<ORD, T, 2>), grd, blk, 0, s, prim, ctx->d_codes, tend, P, FA);
   else
@@ -476,7 +484,7 @@ static CombineParams combine_params(pu_ctx *ctx) {
   P.relax = ctx->d_relax;
   P.positive_mask = 0;
   for (int tr = 0; tr < ctx->cfg.num_tracers; tr++) if (ctx->cfg.tracer_positive[tr]) P.positive_mask |= 1u << tr;
-  P.stage = 0; P.nrelax = 1; P.dt = 0;
+  P.stage = 0; P.nrelax = 1;
   return P;
 }
 

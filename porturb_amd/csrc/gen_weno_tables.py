@@ -209,10 +209,28 @@ def tv_ldl(ord_):
     return out
 
 
+def _fma_sum(terms):
+    """Sum of products (left to right) as one multiply and explicit fused multiply-adds, so that
+    every kernel rounds it the same way.  terms: (literal or None for 1, expression)."""
+    acc = None
+    for c, x in terms:
+        if acc is None:
+            acc = x if c is None else "%s*%s" % (c, x)
+        elif c is None:
+            acc = "%s + %s" % (acc, x)
+        else:
+            acc = "fma(%s, %s, %s)" % (c, x, acc)
+    return acc if acc is not None else "T(0)"
+
+
 def _diff_expr(coefs, var):
     """Straight-line sum of the nonzero terms c*var[i] (left to right)."""
-    terms = ["T(%s)*%s[%d]" % (lit(c), var, i) for i, c in enumerate(coefs) if c != 0]
-    return " + ".join(terms) if terms else "T(0)"
+    return _fma_sum([("T(%s)" % lit(c), "%s[%d]" % (var, i)) for i, c in enumerate(coefs) if c != 0])
+
+
+def _plain_expr(coefs, var):
+    """Straight-line sum of the nonzero terms c*var[i] (left to right), for the compiler to fuse."""
+    return " + ".join("T(%s)*%s[%d]" % (lit(c), var, i) for i, c in enumerate(coefs) if c != 0)
 
 
 def face_differences(ord_, side):
@@ -250,19 +268,25 @@ def emit_ops(path):
             n = N - 1
             terms = []
             for k in range(n):
-                comb = "d[%d]" % (m + k)
-                for j in range(k + 1, n):
-                    if L[j][k] != 0:
-                        comb += " + T(%s)*d[%d]" % (lit(L[j][k]), m + j)
-                out.append("    const T c%d_%d = %s;" % (m, k, comb))
-                terms.append("T(%s)*(c%d_%d*c%d_%d)" % (lit(Dk[k]), m, k, m, k))
-            out.append("    TV[%d] = %s;" % (m, " + ".join(terms)))
+                comb = [(None, "d[%d]" % (m + k))]
+                comb += [("T(%s)" % lit(L[j][k]), "d[%d]" % (m + j)) for j in range(k + 1, n) if L[j][k] != 0]
+                out.append("    const T c%d_%d = %s;" % (m, k, _fma_sum(comb)))
+                coef = None if Dk[k] == 1 else "T(%s)" % lit(Dk[k])
+                terms.append((coef, "(c%d_%d*c%d_%d)" % (m, k, m, k)))
+            out.append("    TV[%d] = %s;" % (m, _fma_sum(terms)))
         out.append("  }")
         for side in ("L", "R"):
             # e[m]: candidate m's value at the face minus the cell average
             out.append("  template <class T> __device__ static __forceinline__ void edge%s(const T *d, T *e) {" % side)
             for m, row in enumerate(face_differences(ord_, side)):
                 out.append("    e[%d] = %s;" % (m, _diff_expr(row, "d")))
+            out.append("  }")
+            # the candidates' face values combined with weights w, and the full-stencil value
+            out.append("  template <class T> __device__ static __forceinline__ T comb%s(const T *s, const T *w) {" % side)
+            out.append("    return %s;" % " + ".join("(%s)*w[%d]" % (_plain_expr(t["face"][side][m], "s"), m) for m in range(S)))
+            out.append("  }")
+            out.append("  template <class T> __device__ static __forceinline__ T lin%s(const T *s) {" % side)
+            out.append("    return %s;" % _plain_expr(t["lin"][side], "s"))
             out.append("  }")
             out.append("  __device__ static __forceinline__ constexpr double ideal%s(int m) {" % side)
             out.append("    constexpr double d[%d] = {%s};" % (S, ",".join(lit(v) for v in t["ideal"][side])))

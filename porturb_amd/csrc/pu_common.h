@@ -127,17 +127,16 @@ __device__ __forceinline__ void swizzled_block(unsigned &bx, unsigned &by, unsig
   bz = l / (gridDim.x * gridDim.y);
 }
 
-// Reciprocal of a positive, normal argument: v_rcp_f32 in FP32; in FP64 v_rcp_f64 refined by two
-// Newton steps (about 1 ulp; every call site divides by a positive quantity >= 1e-20).
+// Reciprocal of a positive, normal argument: v_rcp_f32 in FP32; in FP64 v_rcp_f64 (2^-24) refined by
+// one third-order step, r (1 + e + e^2) with e = 1 - x r: its error e^3 is below 2^-70, so the result
+// is as accurate as after two Newton steps with one multiply-add less.
 template <class T> __device__ __forceinline__ T recip(T x) {
   if constexpr (std::is_same<T, float>::value) {
     return __builtin_amdgcn_rcpf(x);
   } else {
-    double r = __builtin_amdgcn_rcp(x);
-    double e = fma(-x, r, 1.0);
-    r = fma(r, e, r);
-    e = fma(-x, r, 1.0);
-    return fma(r, e, r);
+    const double r = __builtin_amdgcn_rcp(x);
+    const double e = fma(-x, r, 1.0);
+    return fma(r, fma(e, e, e), r);
   }
 }
 

@@ -1,18 +1,20 @@
-// sweep_core.h -- the sweep kernels (WENO limiter, Riemann flux, flux divergence and the fused
+// sweep_core.h -- the FP64 sweep kernels (WENO limiter, Riemann flux, flux divergence and the fused
 // stage combination): the x sweep k_sweep_x, the whole-column z sweep k_sweep_zwall, the whole-line
-// y sweep k_sweep_yline and the general y/z segment sweep k_sweep_seg.  dycore_kernels.hip launches
-// them; the FP32 z, y and x instances are compiled in translation units of their own
-// (sweep_zwall_f32.hip, sweep_yline_f32.hip, sweep_x_f32.hip) without loop-invariant code motion of
-// machine code: hoisting the limiter's constants out of the loops costs those kernels registers and
-// waves of occupancy.
+// y sweep k_sweep_yline and the general y/z segment sweep k_sweep_seg, launched by dycore_kernels.hip,
+// with what they share with the FP32 kernels (T = double throughout the kernels here).
 //
 // Every sweep works in two phases.  Phase A reconstructs density, normal velocity and pressure on
-// both faces of a cell and solves the acoustic Riemann problem at its low face.  That fixes the
-// face's upwind side, and phase B reconstructs each transported quantity (transverse velocities,
-// theta, tracers) only there: one value per face instead of two per cell, of which the flux would
-// use one.  A face whose upwind cell is the upper one reads that cell's stencil in reverse order and
-// takes the same right-face expressions, so a wave with both directions runs one code path.
-// With the full limiter that is 7 of 10 fields (4 tracers) at about 0.6 of the operations.
+// both faces of a cell and solves the acoustic Riemann problem at its low face, which fixes the face's
+// upwind side.  Phase B reconstructs each transported quantity (transverse velocities, theta, tracers)
+// only there: one value per face instead of two per cell, of which the flux would use one.  A face
+// whose upwind cell is the upper one reads that cell's stencil in reverse order and takes the same
+// right-face expressions, so a wave with both directions runs one code path.  With the full limiter
+// that is 7 of 10 fields (4 tracers) at 0.6 of the operations.
+//   The kernels are bound by VALU issue (67-70 % of the SIMD cycles; 2900 instructions per cell and
+// sweep of ten fields, 4350 before).  At 1024x1024x128 WENO-9, ms per launch: z 18.1 -> 14.1, y 19.4 ->
+// 14.8, x 22.7 -> 16.3; of it the upwind side 0.84, the register cap with constants left in the loops
+// 0.95, offsets and bases without 64-bit address arithmetic 0.96.
+// FP32 has kernels of its own (sweep_f32_core.h).
 #pragma once
 #include "pu_common.h"
 #include "weno_ops.h"
@@ -65,27 +67,20 @@ __device__ __forceinline__ unsigned reverse_code(unsigned c) {
 // What the limiter needs of a stencil besides the candidates' face values: the (unnormalised)
 // nonlinear weights without their ideal factors, b[m] = 1 / (TV_m^2 + eps) up to a common factor.
 // Candidate values are carried as differences e[m] from the cell's own average sc: a convex
-// combination of them is sc + sum w_m e_m.
+// combination of them is sc + sum w_m e_m.  All multiply-adds of the limiter are explicit: a stencil
+// gives the same value to the last bit in every kernel.
 //
-// FP64 (same mathematics as the reference, WenoLimiter.h gll_1/gll_2, with a few roundings
-// reordered):
+// The mathematics of the reference (WenoLimiter.h gll_1/gll_2) with a few roundings reordered:
 //  * TV normalisation: with tot = sum(TV) > 1e-20 the reference uses TV_m/tot, so
 //    d_m/((TV_m/tot)^2 + 1e-20) = tot^2 * d_m/(TV_m^2 + 1e-20*tot^2); the common factor tot^2
 //    cancels in the weight normalisation, leaving D_m = TV_m^2 + 1e-20*tot^2.  imm_L/imm_R take a
 //    maximum, which commutes with the positive scaling.
 //  * w_m = d_m/D_m normalised equals d_m*P_m / sum_k d_k*P_k with P_m = prod_{j!=m} D_j
 //    (D >= 1e-20*tot^2 keeps products of S-1 factors far from underflow in double).
-// FP32: the normalised TV and one reciprocal per candidate (products would underflow).
 template <int ORD, class T>
 __device__ __forceinline__ void base_weights(T *TV, T tot, unsigned code, T *b) {
+#pragma clang fp contract(off)
   constexpr int S = pu_weno::Ops<ORD>::S;
-  if constexpr (std::is_same<T, float>::value) {
-    if (PU_FLAT_SHORTCUT || tot > T(1.e-20)) {
-      const T r = recip(tot);
-#pragma unroll
-      for (int m = 0; m < S; m++) TV[m] *= r;
-    }
-  }
   if (code & (SC_FIRST | SC_LAST)) {
     T mx = TV[0];
 #pragma unroll
@@ -93,75 +88,76 @@ __device__ __forceinline__ void base_weights(T *TV, T tot, unsigned code, T *b) 
     if (code & SC_FIRST) TV[S - 1] = mx;
     if (code & SC_LAST) TV[0] = mx;
   }
-  if constexpr (std::is_same<T, float>::value) {
+  T D[S];
+  const T eps = PU_FLAT_SHORTCUT || tot > T(1.e-20) ? T(1.e-20) * (tot * tot) : T(1.e-20);
 #pragma unroll
-    for (int m = 0; m < S; m++) b[m] = recip(TV[m] * TV[m] + T(1.e-20));
-  } else {
-    T D[S];
-    const T eps = PU_FLAT_SHORTCUT || tot > T(1.e-20) ? T(1.e-20) * (tot * tot) : T(1.e-20);
-#pragma unroll
-    for (int m = 0; m < S; m++) D[m] = fma(TV[m], TV[m], eps);
-    excl_products<T, S>(D, b);
-  }
+  for (int m = 0; m < S; m++) D[m] = fma(TV[m], TV[m], eps);
+  excl_products<T, S>(D, b);
+}
+
+// The valid stencil point that stands for point q when the points outside [lo, hi] are replaced
+// (lo <= hs <= hi).
+template <int ORD> __device__ __forceinline__ int valid_point(int q, int lo, int hi) {
+  return q <= (ORD - 1) / 2 ? max(q, lo) : min(q, hi);
 }
 
 // Limited face value from the base weights b and the candidates' values e of one side (RIGHT: the
 // face after the cell in stencil order).
 //  * map_rs (k=6, m=3, s=2000) returns A_m/B_m; the renormalised mapped weights are
 //    A_m*Q_m / sum A_k*Q_k with Q_m = prod_{j!=m} B_j, and the one division goes to the face value.
-//    Safe in FP32 up to ord 9: B_m = (w-d)^6 + 2000 (w(1-w))^3 lies in [0.99 d_m^6, 32], and with the
-//    ideal weights of ord <= 9 (>= 1/126) a product of S-1 factors stays above 1e-29 and below 1e6
-//    (ord 11 could reach 1e-42: in FP32 it divides per candidate).
 template <int ORD, class T, bool RIGHT>
 __device__ __forceinline__ T limited_value(const T *b, const T *e, T sc, bool do_map) {
+#pragma clang fp contract(off)
   using O = pu_weno::Ops<ORD>;
   constexpr int S = O::S;
-  T w[S], sum = T(0), dot = T(0);
+  T w[S], ideal[S];
 #pragma unroll
   for (int m = 0; m < S; m++) {
-    w[m] = T(RIGHT ? O::idealR(m) : O::idealL(m)) * b[m];
-    sum += w[m];
+    ideal[m] = T(RIGHT ? O::idealR(m) : O::idealL(m));
+    w[m] = ideal[m] * b[m];
   }
-  const T r = recip(sum);
-  if (!do_map) {
+  T sum = w[0];
 #pragma unroll
-    for (int m = 0; m < S; m++) dot += w[m] * e[m];
-    return fma(dot, r, sc);
-  }
+  for (int m = 1; m < S; m++) sum = fma(ideal[m], b[m], sum);
+  const T r = recip(sum);
+  auto dot = [&]() {
+    T v = w[0] * e[0];
+#pragma unroll
+    for (int m = 1; m < S; m++) v = fma(w[m], e[m], v);
+    return v;
+  };
+  if (!do_map) return fma(dot(), r, sc);
   T A[S], B[S];
 #pragma unroll
   for (int m = 0; m < S; m++) {
-    const T d = T(RIGHT ? O::idealR(m) : O::idealL(m));
-    const T x = w[m] * r;
+    const T d = ideal[m], x = w[m] * r;
     if constexpr (O::use_map_rs) {
-      const T dl = x - d, d2 = dl * dl, t1 = d2 * d2 * d2, ww = fma(-x, x, x), t2 = ww * ww * ww;
+      const T dl = fma(w[m], r, -d), d2 = dl * dl, t1 = d2 * d2 * d2, ww = fma(-x, x, x), t2 = ww * ww * ww;
       B[m] = fma(T(2000), t2, t1);
       A[m] = fma(d, B[m], t1 * dl);
     } else {                                             // map_w (ord 3)
-      B[m] = d * d + (T(1) - T(2) * d) * x;
-      A[m] = x * (d + d * d - T(3) * d * x + x * x);
+      B[m] = fma(T(1) - T(2) * d, x, d * d);
+      A[m] = x * fma(x, x, fma(T(-3) * d, x, fma(d, d, d)));
     }
   }
-  sum = T(0);
-  if constexpr (std::is_same<T, float>::value && ORD > 9) {
+  T Q[S];
+  excl_products<T, S>(B, Q);
 #pragma unroll
-    for (int m = 0; m < S; m++) { w[m] = A[m] * recip(B[m]); sum += w[m]; dot += w[m] * e[m]; }
-  } else {
-    T Q[S];
-    excl_products<T, S>(B, Q);
+  for (int m = 0; m < S; m++) w[m] = A[m] * Q[m];
+  sum = w[0];
 #pragma unroll
-    for (int m = 0; m < S; m++) { w[m] = A[m] * Q[m]; sum += w[m]; dot += w[m] * e[m]; }
-  }
-  return fma(dot, recip(sum), sc);
+  for (int m = 1; m < S; m++) sum = fma(A[m], Q[m], sum);
+  return fma(dot(), recip(sum), sc);
 }
 
 // The linear (ideal-weight) reconstruction.
 template <int ORD, class T, bool RIGHT>
 __device__ __forceinline__ T linear_value(const T *e, T sc) {
+#pragma clang fp contract(off)
   using O = pu_weno::Ops<ORD>;
-  T dot = T(0);
+  T dot = T(RIGHT ? O::idealR(0) : O::idealL(0)) * e[0];
 #pragma unroll
-  for (int m = 0; m < O::S; m++) dot += T(RIGHT ? O::idealR(m) : O::idealL(m)) * e[m];
+  for (int m = 1; m < O::S; m++) dot = fma(T(RIGHT ? O::idealR(m) : O::idealL(m)), e[m], dot);
   return sc + dot;
 }
 
@@ -203,7 +199,7 @@ __device__ __forceinline__ void cell_values(const T *s, unsigned code, bool use_
   qR = limited_value<ORD, T, true>(b, eR, sc, do_map);
 }
 
-// The value at the face after the cell, in the order the stencil is read.
+// FP64: the value at the face after the cell, in the order the stencil is read.
 template <int ORD, class T>
 __device__ __forceinline__ T face_value(const T *s, unsigned code, bool use_weno) {
   using O = pu_weno::Ops<ORD>;
@@ -223,6 +219,9 @@ __device__ __forceinline__ T face_value(const T *s, unsigned code, bool use_weno
 template <class T, class OFF> __device__ __forceinline__ T load_at(const T *base, OFF off) {
   return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + off);
 }
+template <class T> __device__ __forceinline__ void store_at(T *base, unsigned off, T v) {
+  *reinterpret_cast<T *>(reinterpret_cast<char *>(base) + off) = v;
+}
 
 // A cell's stencil in memory order; `base`: its first point for lane offset 0, sstride its step
 // (uniform).  clamp: replace immersed points (transverse velocities and pressure).
@@ -232,89 +231,129 @@ __device__ __forceinline__ void load_stencil(const T *base, long long sstride, O
     const int lo = code & SC_LO, hi = ORD - 1 - (int)((code & SC_GAP) >> 4);
 #pragma unroll
     for (int q = 0; q < ORD; q++)
-      s[q] = load_at<T, OFF>(base, off + (OFF)clampi(q, lo, hi) * (OFF)(sstride * (long long)sizeof(T)));
+      s[q] = load_at<T, OFF>(base, off + (OFF)valid_point<ORD>(q, lo, hi) * (OFF)(sstride * (long long)sizeof(T)));
   } else {
 #pragma unroll
     for (int q = 0; q < ORD; q++) s[q] = load_at<T, OFF>(base + q * sstride, off);
   }
 }
 
-// The stencil of a face's upwind cell, read from the upwind end: point q at off0 + q*step.
+// The stencil of a face's upwind cell, read from the upwind end.  The points' offsets are the same
+// for every transported quantity, so they are worked out once per face and a load costs no address
+// arithmetic; the transverse velocities (the first two quantities) take them with immersed points
+// replaced, plain() gives the others theirs.
 template <int ORD, class OFF> struct UpwindStencil {
-  OFF off0, step;
+  OFF off[ORD], off0, step;
   unsigned code;                   // in reading order
-  // own: the lane's offset of its own cell's first stencil point minus one step (the lower
-  // neighbour's first point); left: the lower neighbour is upwind; lower/own_code: stencil codes
-  __device__ __forceinline__ void setup(OFF own, OFF stride, bool left, unsigned lower_code, unsigned own_code) {
-    off0 = left ? own : own + (OFF)ORD * stride;
+  // lane: the lane's offset of the lower neighbour's first point; left: the lower neighbour is
+  // upwind; lower_code / own_code: stencil codes of the two cells
+  __device__ __forceinline__ void setup(OFF lane, OFF stride, bool left, unsigned lower_code, unsigned own_code) {
+    off0 = left ? lane : lane + (OFF)ORD * stride;
     step = left ? stride : (OFF)0 - stride;
     code = left ? lower_code : (own_code ? reverse_code(own_code) : 0u);
-  }
-  template <class T> __device__ __forceinline__ void load(const T *base, bool clamp, T *s) const {
-    if (clamp && (code & SC_CLAMP)) {
+    plain();
+    if (code & SC_CLAMP) {
       const int lo = code & SC_LO, hi = ORD - 1 - (int)((code & SC_GAP) >> 4);
 #pragma unroll
-      for (int q = 0; q < ORD; q++) s[q] = load_at<T, OFF>(base, off0 + (OFF)clampi(q, lo, hi) * step);
-    } else {
-#pragma unroll
-      for (int q = 0; q < ORD; q++) s[q] = load_at<T, OFF>(base, off0 + (OFF)q * step);
+      for (int q = 0; q < ORD; q++) off[q] = off0 + (OFF)valid_point<ORD>(q, lo, hi) * step;
     }
+  }
+  __device__ __forceinline__ void plain() {
+    off[0] = off0;
+#pragma unroll
+    for (int q = 1; q < ORD; q++) off[q] = off[q - 1] + step;
+  }
+  template <class T> __device__ __forceinline__ void load(const T *base, T *s) const {
+#pragma unroll
+    for (int q = 0; q < ORD; q++) s[q] = load_at<T, OFF>(base, off[q]);
   }
 };
 
-// acoustic upwind state of one face (dynamics_rk.h:640-651): mass flux, pressure, upwind side
-template <class T> struct Upw { T ru, p; bool left; };
+// acoustic upwind state of one face (dynamics_rk.h:640-651): mass flux, pressure, upwind side.  The
+// multiply-adds are written out, here and in carried(): every kernel then rounds a face's fluxes
+// the same way, whatever code surrounds them.
+template <class T> struct Upw {
+  T ru, p;
+  bool left;
+  __device__ __forceinline__ T momentum(T uL, T uR) const { return fma(ru, left ? uL : uR, p); }
+};
 
 template <class T>
 __device__ __forceinline__ Upw<T> riemann(T rL, T uL, T pL, T rR, T uR, T pR, T hr) {
-  rL += hr; rR += hr;
-  const T cs = T(350.);
-  T ruL = uL * rL, ruR = uR * rR;
+#pragma clang fp contract(off)
+  const T ruL = uL * (rL + hr), ruR = uR * (rR + hr);
   Upw<T> u;
-  u.p = T(0.5) * (pL + pR - cs * (ruR - ruL));
-  u.ru = T(0.5) * (ruL + ruR - (pR - pL) * T(1. / 350.));
+  u.p = T(0.5) * fma(T(-350.), ruR - ruL, pL + pR);
+  u.ru = T(0.5) * fma(T(-1. / 350.), pR - pL, ruL + ruR);
   u.left = u.ru > 0;
   return u;
 }
 
-// Transported quantity b of a sweep along DIR: its primitive-field and flux index and whether its
-// stencil replaces immersed points.
-template <int DIR> __device__ __forceinline__ void transported(int b, int &l, int &fidx, bool &clamp) {
-  clamp = b < 2;
-  if (b == 0) l = fidx = DIR == 0 ? idV : idU;
-  else if (b == 1) l = fidx = DIR == 2 ? idV : idW;
-  else if (b == 2) l = fidx = idT;
-  else { l = NUM_STATE + 1 + (b - 3); fidx = NUM_STATE + (b - 3); }
+// Flux of a transported value: rounded by itself, never fused into the divergence that follows, so
+// that a face's two cells see the same flux and every kernel computes the same tendencies.
+template <class T> __device__ __forceinline__ T carried(T ru, T v) {
+#pragma clang fp contract(off)
+  return ru * v;
 }
 
+// The transported quantities of a sweep in their order: the transverse velocities (stencils with
+// immersed points replaced), theta (its hydrostatic part is added at the face), the tracers.  Calls
+// f(is theta, primitive field, conserved field, quantity) for each.  PEEL: each of the first three
+// from its own call site, so that the code for each holds only its own cases; the x sweep, whose
+// stage combination differs by field, gains by it, the chunk-walking sweeps lose registers.
+template <int DIR, bool PEEL, class US, class F> __device__ __forceinline__ void transport_all(US &us, int ntr, F &&f) {
+  constexpr int first = DIR == 0 ? idV : idU, second = DIR == 2 ? idV : idW;
+  if constexpr (PEEL) {
+    f(false, first, first, 0);
+    f(false, second, second, 1);
+    us.plain();
+    f(true, (int)idT, (int)idT, 2);
+    for (int tr = 0; tr < ntr; tr++) f(false, NUM_STATE + 1 + tr, NUM_STATE + tr, 3 + tr);
+  } else {
+    for (int b = 0; b < 3 + ntr; b++) {
+      if (b == 2) us.plain();
+      const int l = b == 0 ? first : (b == 1 ? second : (b == 2 ? idT : NUM_STATE + b - 2));
+      f(b == 2, l, b < 3 ? l : NUM_STATE + b - 3, b);
+    }
+  }
+}
+
+// Block of a chunk-walking sweep: CH_BX cells across, CH_BS along (at 512x512x128 WENO-9 in FP64 per
+// launch 8x32 ran 3.42 (z) and 3.57 ms (y), 16x16 3.45 and 3.76, 4x64 3.7 and 3.6, 16x32 3.9 and 4.1;
+// FP32 likewise).
+constexpr int CH_BX = 8, CH_BS = 32;
+
+// FP64 sweeps: at most 96 VGPRs (5 waves per SIMD), which they fit without spills up to WENO-9
+// (WENO-11 spills up to 30 there and takes 4 waves)
+__host__ __device__ constexpr int f64_waves(int ord) { return ord <= 9 ? 5 : 4; }
 constexpr int SW_NQ = 5 + PU_MAX_TRACERS;     // fluxes of a face: mass, normal momentum, transported
 
 // Whether the lane offsets of a line kernel (a chunk of 32 cells and its halo along the sweep) fit
 // 32 bits: sstride = elements between cells along the sweep.
 template <class T> static inline bool offsets_fit(long long sstride, int hp) {
-  return (32 + 2 * hp + 2) * sstride * (long long)sizeof(T) + 4096 < (1LL << 32);
+  return (CH_BS + 2 * hp + 2) * sstride * (long long)sizeof(T) + 4096 < (1LL << 32);
 }
 
 // ------------------------------------------------------------------------------------------------
 // z sweep between solid walls (the first sweep of a stage, writing the tendencies): one block per
-// 8 columns walks the whole column in chunks of 32 cells, every thread owning one cell per chunk.
+// BX columns walks the whole column in chunks of BS cells, every thread owning one cell per chunk.
 // Walls need no neighbour cells (the wall faces take the adjacent cell's own values,
 // dynamics_rk.h:864-888), and the face between two chunks takes the lower chunk's top values from
 // a small LDS carry, so no cell is reconstructed twice (the segment kernel reconstructs 160 cells
-// for each 128-level column).  Thread (x, t) of chunk q owns cell r = 32q + t: it computes the
+// for each 128-level column).  Thread (x, t) of chunk q owns cell r = BS q + t: it computes the
 // face below r (r = 0: the bottom wall) and finishes the tendency of cell r-1; the thread of the
 // top cell also finishes its own tendency with the top wall face, whose Riemann state with w = 0
 // on both sides and equal left/right values is exactly mass flux 0 and pressure p (every other
 // flux through it is 0).  Otherwise the arithmetic of k_sweep_seg<ORD, T, 2>, operand for operand.
 // A face's fluxes alternate between two LDS buffers, so a transported quantity costs one barrier.
 // ------------------------------------------------------------------------------------------------
-constexpr int ZW_BX = 8, ZW_BS = 32;
 
 template <int ORD, class T>
-__global__ __launch_bounds__(ZW_BX * ZW_BS) void k_sweep_zwall(const T *__restrict__ prim,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(f64_waves(ORD))))
+void k_sweep_zwall(const T *__restrict__ prim,
                                                              const uint16_t *__restrict__ codes, T *__restrict__ tend,
                                                              SweepParams P) {
-  constexpr int BX = ZW_BX, BS = ZW_BS, NT = BX * BS, hs = (ORD - 1) / 2;
+  constexpr int BX = CH_BX, BS = CH_BS, NT = BX * BS, hs = (ORD - 1) / 2;
   __shared__ T sQ[3][NT], sA[2][NT], sB[2][NT];
   __shared__ T carQ[2][3][BX], carF[2][SW_NQ][BX];          // by chunk parity
 
@@ -326,9 +365,10 @@ __global__ __launch_bounds__(ZW_BX * ZW_BS) void k_sweep_zwall(const T *__restri
   const long long plane = P.nxh * P.nyh, cplane = (long long)P.nx * P.ny;
   const unsigned stride = (unsigned)(plane * (long long)sizeof(T));
   const unsigned lane = (unsigned)((ty * plane + tx) * (long long)sizeof(T));
+  const unsigned clane = (unsigned)((ty * cplane + tx) * (long long)sizeof(T));    // tendencies, one cell below
+  const unsigned ctop = clane + (unsigned)(cplane * (long long)sizeof(T));
   const T rd = (T)P.rd;
   const int nchunk = (nz + BS - 1) / BS;
-  const int nB = 3 + P.ntr;
 
   for (int q = 0; q < nchunk; q++) {
     const int r = q * BS + ty;
@@ -339,10 +379,12 @@ __global__ __launch_bounds__(ZW_BX * ZW_BS) void k_sweep_zwall(const T *__restri
     const int pin = (q + 1) & 1, pout = q & 1;
     // first stencil point of the cell below the chunk's first one, at the block's first column
     const T *row = prim + ((long long)(q * BS) * P.nyh + (j + P.hp)) * P.nxh + (P.ox + (int)bx * BX);
-    const long long cid = ((long long)r * P.ny + j) * P.nx + i;
+    // cell of lane (0, 0) one level below the chunk, in the cell arrays
+    const long long below = ((long long)(q * BS - 1) * P.ny + j) * P.nx + (int)bx * BX;
     unsigned own = 0, lower = 0;
     T hr = 0, ht = 0;
     if (valid) {
+      const long long cid = ((long long)r * P.ny + j) * P.nx + i;
       own = codes[cid];
       if (r > 0) lower = codes[cid - cplane];
       hr = (T)P.hy_re[r];
@@ -374,7 +416,7 @@ __global__ __launch_bounds__(ZW_BX * ZW_BS) void k_sweep_zwall(const T *__restri
       if (bot) { rL = rR; uL = 0; uR = 0; pL = pR; }
       up = riemann(rL, uL, pL, rR, uR, pR, hr);
       Fr = up.ru;
-      Fu = up.ru * (up.left ? uL : uR) + up.p;
+      Fu = up.momentum(uL, uR);
     }
     sA[0][lin] = Fr; sA[1][lin] = Fu;
     __syncthreads();
@@ -382,12 +424,12 @@ __global__ __launch_bounds__(ZW_BX * ZW_BS) void k_sweep_zwall(const T *__restri
       if (r > 0) {
         const T Fr0 = ty > 0 ? sA[0][lin - BX] : carF[pin][0][tx];
         const T Fu0 = ty > 0 ? sA[1][lin - BX] : carF[pin][1][tx];
-        tend[(long long)idR * P.n3 + cid - cplane] = -(Fr - Fr0) * rd;
-        tend[(long long)idW * P.n3 + cid - cplane] = -(Fu - Fu0) * rd;
+        store_at(tend + ((long long)idR * P.n3 + below), clane, -(Fr - Fr0) * rd);
+        store_at(tend + ((long long)idW * P.n3 + below), clane, -(Fu - Fu0) * rd);
       }
       if (top) {
-        tend[(long long)idR * P.n3 + cid] = -(T(0) - Fr) * rd;
-        tend[(long long)idW * P.n3 + cid] = -(qRp - Fu) * rd;
+        store_at(tend + ((long long)idR * P.n3 + below), ctop, -(T(0) - Fr) * rd);
+        store_at(tend + ((long long)idW * P.n3 + below), ctop, -(qRp - Fu) * rd);
       }
     }
     if (carry_out) {
@@ -395,33 +437,33 @@ __global__ __launch_bounds__(ZW_BX * ZW_BS) void k_sweep_zwall(const T *__restri
       carF[pout][0][tx] = Fr; carF[pout][1][tx] = Fu;
     }
 
-    // ---- phase B: the transported quantities on the face's upwind side, one at a time ----
+    // ---- phase B: the transported quantities, one at a time ----
+    // tendency of the cell below the face (and of the top cell) from the fluxes in sF
+    auto finish = [&](const T *sF, int fidx, int b, T F) {
+      if (valid) {
+        T *tp = tend + ((long long)fidx * P.n3 + below);
+        if (r > 0) store_at(tp, clane, -(F - (ty > 0 ? sF[lin - BX] : carF[pin][2 + b][tx])) * rd);
+        if (top) store_at(tp, ctop, -(T(0) - F) * rd);
+      }
+      if (carry_out) carF[pout][2 + b][tx] = F;
+    };
     UpwindStencil<ORD, unsigned> us;
     us.setup(lane, stride, up.left && !bot, lower, own);
     const bool weno_up = P.weno_all || (us.code & SC_ANY);
-    for (int b = 0; b < nB; b++) {
-      int l, fidx;
-      bool clamp;
-      transported<2>(b, l, fidx, clamp);
+    transport_all<2, false>(us, P.ntr, [&](bool theta, int l, int fidx, int b) {
       T F = 0;
       if (valid) {
         T s[ORD];
-        us.load(row + (long long)l * P.nh, clamp, s);
+        us.load(row + (long long)l * P.nh, s);
         T v = face_value<ORD, T>(s, us.code, weno_up);
-        if (bot && l == idT) v = 0;
-        if (l == idT) v += ht;
-        F = up.ru * v;
+        if (theta) v = (bot ? T(0) : v) + ht;
+        F = carried(up.ru, v);
       }
       T *sF = sB[b & 1];
       sF[lin] = F;
       __syncthreads();
-      if (valid) {
-        T *tp = tend + (long long)fidx * P.n3 + cid;
-        if (r > 0) tp[-cplane] = -(F - (ty > 0 ? sF[lin - BX] : carF[pin][2 + b][tx])) * rd;
-        if (top) *tp = -(T(0) - F) * rd;
-      }
-      if (carry_out) carF[pout][2 + b][tx] = F;
-    }
+      finish(sF, fidx, b, F);
+    });
   }
 }
 
@@ -430,7 +472,8 @@ struct CombineParams {
   int nx, ny, nz, hs, ntr, stage, nrelax, enable_gravity, coriolis;
   int sim2d;                        // ny == 1: the V tendency is zero (dynamics_rk.h:716)
   long long n3;
-  double dt, grav, fcor;
+  double cu, cs, ct;                // the stage's combination: cu*U + cs*Us + ct*tendency
+  double grav, fcor;
   const double *hy_r, *hy_t;        // cells
   const double *relax;              // [n3]
   unsigned int positive_mask;       // bit tr set if tracer tr is positive-definite
@@ -459,82 +502,80 @@ __device__ __forceinline__ void store_cons(ST *U, ST *Ulo, int l, long long id, 
   }
 }
 
-// ------------------------------------------------------------------------------------------------
-// SSPRK3 stage combination of one conserved field of one cell (time_step_rk_3_3,
-// dynamics_rk.h:279-367): gravity and Coriolis sources, the stage's convex combination, the
-// positivity clip of the last stage and nrelax immersed relaxations (enforce_immersed_boundaries,
-// :370-473).  rho_in, u_in, v_in are the stage-input state of the cell, read before any field of the
-// cell is overwritten (stage 1 writes Us in place).
-// ------------------------------------------------------------------------------------------------
 template <class ST> struct FuseArgs {
   ST *U, *Ulo, *Us, *Uslo;
   CombineParams C;
 };
 
-// un, us: the field's values in U and (stages 1, 2) Us, read by the caller ahead of time
-template <class ST>
-__device__ __forceinline__ void combine_field_v(const FuseArgs<ST> &F, int l, long long id, double tn, double un,
-                                                double us, double rho_in, double u_in, double v_in, double mult,
-                                                double tr_r, double tr_rt) {
-  const CombineParams &P = F.C;
-  if (l == idV && P.sim2d) tn = 0.;
-  if (l == idW && P.enable_gravity) tn += -P.grav * (rho_in - tr_r);
-  if (P.coriolis && l == idU) tn += P.fcor * v_in;
-  if (P.coriolis && l == idV) tn -= P.fcor * u_in;
-  double v;
-  if (P.stage == 0) {
-    v = un + P.dt * tn;
-  } else if (P.stage == 1) {
-    v = (3. / 4.) * un + (1. / 4.) * us + (1. / 4.) * P.dt * tn;
-  } else {
-    v = (1. / 3.) * un + (2. / 3.) * us + (2. / 3.) * P.dt * tn;
-  }
-  bool positive = l >= NUM_STATE && ((P.positive_mask >> (l - NUM_STATE)) & 1u);
-  if (P.stage == 2 && positive) v = fmax(0., v);
-  double target = l == idR ? tr_r : (l == idT ? tr_rt : 0.);
-  for (int r = 0; r < P.nrelax; r++) {
-    v = v + (target - v) * mult;
-    if (positive) v = fmax(0., v);
-  }
-  if (P.stage == 2) store_cons(F.U, F.Ulo, l, id, P.n3, v);
-  else store_cons(F.Us, F.Uslo, l, id, P.n3, v);
+// The same in double for cells addressed as a uniform cell number plus the lane's byte offset.
+__device__ __forceinline__ double load_cons_at(const double *U, int l, long long cell, unsigned lane, long long n3) {
+  return load_at<double, unsigned>(U + ((long long)l * n3 + cell), lane);
 }
 
+// The stage-input state of a cell the combination needs, read before any field of the cell is
+// overwritten (stage 1 writes Us in place), and its relaxation multiplier and targets.
+struct StageIn { double rho, u, v, mult, trr, trt; };
+
 template <class ST>
-__device__ __forceinline__ void stage_inputs(const FuseArgs<ST> &F, long long id, int k, double &rho_in, double &u_in,
-                                             double &v_in, double &mult, double &tr_r, double &tr_rt) {
+__device__ __forceinline__ StageIn stage_inputs(const FuseArgs<ST> &F, long long id, int k) {
   const CombineParams &P = F.C;
   const ST *Sin = P.stage == 0 ? F.U : F.Us;
   const ST *Sinlo = P.stage == 0 ? F.Ulo : F.Uslo;
-  rho_in = load_cons(Sin, Sinlo, idR, id, P.n3);
-  u_in = P.coriolis ? load_cons(Sin, Sinlo, idU, id, P.n3) : 0.;
-  v_in = P.coriolis ? load_cons(Sin, Sinlo, idV, id, P.n3) : 0.;
-  mult = P.relax[id];
-  tr_r = P.hy_r[P.hs + k];
-  tr_rt = P.hy_r[P.hs + k] * P.hy_t[P.hs + k];
+  StageIn S;
+  S.rho = load_cons(Sin, Sinlo, idR, id, P.n3);
+  S.u = P.coriolis ? load_cons(Sin, Sinlo, idU, id, P.n3) : 0.;
+  S.v = P.coriolis ? load_cons(Sin, Sinlo, idV, id, P.n3) : 0.;
+  S.mult = P.relax[id];
+  S.trr = P.hy_r[P.hs + k];
+  S.trt = P.hy_r[P.hs + k] * P.hy_t[P.hs + k];
+  return S;
 }
 
 // ------------------------------------------------------------------------------------------------
-// y sweep along periodic lines (adds to the tendencies): one block walks 8 whole lines in chunks of
-// 32 cells, every thread owning one cell per chunk, so no cell is reconstructed twice (the segment
+// SSPRK3 stage combination of one conserved field of one cell (time_step_rk_3_3,
+// dynamics_rk.h:279-367): gravity and Coriolis sources, the stage's convex combination, the
+// positivity clip of the last stage and nrelax immersed relaxations (enforce_immersed_boundaries,
+// :370-473).  tn: the field's tendency; un, us: its values in U and (stages 1, 2) Us.
+// ------------------------------------------------------------------------------------------------
+__device__ __forceinline__ double combine_value(const CombineParams &P, int l, double tn, double un, double us,
+                                                const StageIn &S) {
+  if (l == idV && P.sim2d) tn = 0.;
+  if (l == idW && P.enable_gravity) tn += -P.grav * (S.rho - S.trr);
+  if (P.coriolis && l == idU) tn += P.fcor * S.v;
+  if (P.coriolis && l == idV) tn -= P.fcor * S.u;
+  double v = fma(P.ct, tn, fma(P.cu, un, P.cs * us));
+  // a cell outside immersed regions has multiplier 0: its relaxations change nothing but the clip,
+  // which is idempotent (the last stage clips before the first relaxation as well)
+  const bool positive = l >= NUM_STATE && ((P.positive_mask >> (l - NUM_STATE)) & 1u);
+  if (S.mult != 0.) {
+    const double target = l == idR ? S.trr : (l == idT ? S.trt : 0.);
+    if (P.stage == 2 && positive) v = fmax(0., v);
+    for (int r = 0; r < P.nrelax; r++) {
+      v = v + (target - v) * S.mult;
+      if (positive) v = fmax(0., v);
+    }
+  } else if (positive) {
+    v = fmax(0., v);
+  }
+  return v;
+}
+
+// ------------------------------------------------------------------------------------------------
+// y sweep along periodic lines (adds to the tendencies): one block walks BX whole lines in chunks of
+// BS cells, every thread owning one cell per chunk, so no cell is reconstructed twice (the segment
 // kernel reconstructs 1120 cells for each 1024-cell line).  Thread t of chunk q owns cell
-// r = 32q + t: it computes the face below it and finishes the tendency of cell r-1; the face between
+// r = BS q + t: it computes the face below it and finishes the tendency of cell r-1; the face between
 // two chunks takes the lower chunk's top values from an LDS carry.  The thread of cell 0
 // reconstructs the upper values of cell -1 (cell N-1 seen through the periodic halo: three one-sided
 // reconstructions once per line) and so has the periodic face from the start; its fluxes are kept
 // in LDS for cell N-1, whose upper face it is.  Otherwise the arithmetic of k_sweep_seg<ORD, T, 1>.
 // ------------------------------------------------------------------------------------------------
-constexpr int YL_BX = 8, YL_BS = 32;
 
-// FP32: at most 72 VGPRs (7 waves per SIMD)
-#ifndef PU_YLINE_F32_WAVES
-#define PU_YLINE_F32_WAVES 7
-#endif
 template <int ORD, class T>
-__global__ __launch_bounds__(YL_BX * YL_BS)
-__attribute__((amdgpu_waves_per_eu(std::is_same<T, float>::value ? PU_YLINE_F32_WAVES : 1)))
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(f64_waves(ORD))))
 void k_sweep_yline(const T *__restrict__ prim, const uint16_t *__restrict__ codes, T *__restrict__ tend, SweepParams P) {
-  constexpr int BX = YL_BX, BS = YL_BS, NT = BX * BS, hs = (ORD - 1) / 2;
+  constexpr int BX = CH_BX, BS = CH_BS, NT = BX * BS, hs = (ORD - 1) / 2;
   __shared__ T sQ[3][NT], sA[2][NT], sB[2][NT];
   __shared__ T carQ[2][3][BX], carF[2][SW_NQ][BX];          // by chunk parity
   __shared__ T firstF[SW_NQ][BX];                            // the periodic face
@@ -546,10 +587,11 @@ void k_sweep_yline(const T *__restrict__ prim, const uint16_t *__restrict__ code
   const bool col_ok = i < P.nx;
   const unsigned stride = (unsigned)(P.nxh * (long long)sizeof(T));
   const unsigned lane = (unsigned)((ty * P.nxh + tx) * (long long)sizeof(T));
+  const unsigned clane = (unsigned)((ty * (long long)P.nx + tx) * (long long)sizeof(T));   // tendencies, one cell below
+  const unsigned clast = clane + (unsigned)(P.nx * (long long)sizeof(T));
   const T rd = (T)P.rd;
   const T hr = (T)P.hy_rc[P.hs + k], ht = (T)P.hy_tc[P.hs + k];
   const int nchunk = (N + BS - 1) / BS;
-  const int nB = 3 + P.ntr;
   const long long cline = (long long)k * P.ny * P.nx + i;      // cell 0 of the thread's line
 
   for (int q = 0; q < nchunk; q++) {
@@ -559,15 +601,24 @@ void k_sweep_yline(const T *__restrict__ prim, const uint16_t *__restrict__ code
     const bool first = r == 0, last = valid && r == N - 1;
     const int pin = (q + 1) & 1, pout = q & 1;
     const T *row = prim + ((long long)(k + P.hp) * P.nyh + q * BS) * P.nxh + (P.ox + (int)bx * BX);
-    const long long cid = cline + (long long)r * P.nx;
+    // cell of lane (0, 0) one row below the chunk, in the cell arrays
+    const long long below = ((long long)k * P.ny + (q * BS - 1)) * P.nx + (int)bx * BX;
     unsigned own = 0, lower = 0;
     if (valid) {
+      const long long cid = cline + (long long)r * P.nx;
       own = codes[cid];
       lower = codes[first ? cline + (long long)(N - 1) * P.nx : cid - P.nx];
     }
     const bool weno = P.weno_all || (own & SC_ANY);
     // the incoming tendencies are loaded ahead of the reconstructions that complete them
-    auto incoming = [&](int fidx) { return valid && r > 0 ? tend[(long long)fidx * P.n3 + cid - P.nx] : T(0); };
+    auto incoming = [&](int fidx) {
+      return valid && r > 0 ? load_at<T, unsigned>(tend + ((long long)fidx * P.n3 + below), clane) : T(0);
+    };
+    auto finish = [&](int fidx, T v) { store_at(tend + ((long long)fidx * P.n3 + below), clane, v); };
+    auto finish_last = [&](int fidx, T v) {
+      T *tp = tend + ((long long)fidx * P.n3 + below);
+      store_at(tp, clast, load_at<T, unsigned>(tp, clast) + v);
+    };
 
     // ---- phase A: density, v, pressure -> acoustic upwinding ----
     T qLr = 0, qRr = 0, qLu = 0, qRu = 0, qLp = 0, qRp = 0;
@@ -600,7 +651,7 @@ void k_sweep_yline(const T *__restrict__ prim, const uint16_t *__restrict__ code
       else if (ty > 0) { rL = sQ[0][lin - BX]; uL = sQ[1][lin - BX]; pL = sQ[2][lin - BX]; }
       up = riemann(rL, uL, pL, qLr, qLu, qLp, hr);
       Fr = up.ru;
-      Fu = up.ru * (up.left ? uL : qLu) + up.p;
+      Fu = up.momentum(uL, qLu);
     }
     sA[0][lin] = Fr; sA[1][lin] = Fu;
     if (first) { firstF[0][tx] = Fr; firstF[1][tx] = Fu; }
@@ -608,44 +659,43 @@ void k_sweep_yline(const T *__restrict__ prim, const uint16_t *__restrict__ code
     if (valid && r > 0) {
       const T Fr0 = ty > 0 ? sA[0][lin - BX] : carF[pin][0][tx];
       const T Fu0 = ty > 0 ? sA[1][lin - BX] : carF[pin][1][tx];
-      tend[(long long)idR * P.n3 + cid - P.nx] = tr0 + -(Fr - Fr0) * rd;
-      tend[(long long)idV * P.n3 + cid - P.nx] = tu0 + -(Fu - Fu0) * rd;
+      finish(idR, tr0 + -(Fr - Fr0) * rd);
+      finish(idV, tu0 + -(Fu - Fu0) * rd);
     }
     if (last) {
-      tend[(long long)idR * P.n3 + cid] += -(firstF[0][tx] - Fr) * rd;
-      tend[(long long)idV * P.n3 + cid] += -(firstF[1][tx] - Fu) * rd;
+      finish_last(idR, -(firstF[0][tx] - Fr) * rd);
+      finish_last(idV, -(firstF[1][tx] - Fu) * rd);
     }
     if (carry_out) {
       carQ[pout][0][tx] = qRr; carQ[pout][1][tx] = qRu; carQ[pout][2][tx] = qRp;
       carF[pout][0][tx] = Fr; carF[pout][1][tx] = Fu;
     }
 
-    // ---- phase B: the transported quantities on the face's upwind side, one at a time ----
+    // ---- phase B: the transported quantities, one at a time ----
+    auto complete = [&](const T *sF, int fidx, int b, T F, T t0) {
+      if (valid && !first) finish(fidx, t0 + -(F - (ty > 0 ? sF[lin - BX] : carF[pin][2 + b][tx])) * rd);
+      if (last) finish_last(fidx, -(firstF[2 + b][tx] - F) * rd);
+      if (carry_out) carF[pout][2 + b][tx] = F;
+    };
     UpwindStencil<ORD, unsigned> us;
     us.setup(lane, stride, up.left, lower, own);
     const bool weno_up = P.weno_all || (us.code & SC_ANY);
-    for (int b = 0; b < nB; b++) {
-      int l, fidx;
-      bool clamp;
-      transported<1>(b, l, fidx, clamp);
+    transport_all<1, false>(us, P.ntr, [&](bool theta, int l, int fidx, int b) {
       const T t0 = incoming(fidx);
       T F = 0;
       if (valid) {
         T s[ORD];
-        us.load(row + (long long)l * P.nh, clamp, s);
+        us.load(row + (long long)l * P.nh, s);
         T v = face_value<ORD, T>(s, us.code, weno_up);
-        if (l == idT) v += ht;
-        F = up.ru * v;
+        if (theta) v += ht;
+        F = carried(up.ru, v);
       }
       T *sF = sB[b & 1];
       sF[lin] = F;
       if (first) firstF[2 + b][tx] = F;
       __syncthreads();
-      if (valid && r > 0)
-        tend[(long long)fidx * P.n3 + cid - P.nx] = t0 + -(F - (ty > 0 ? sF[lin - BX] : carF[pin][2 + b][tx])) * rd;
-      if (last) tend[(long long)fidx * P.n3 + cid] += -(firstF[2 + b][tx] - F) * rd;
-      if (carry_out) carF[pout][2 + b][tx] = F;
-    }
+      complete(sF, fidx, b, F, t0);
+    });
   }
 }
 
@@ -676,12 +726,9 @@ template <int CTRL, class T> __device__ __forceinline__ T wave_shift_value(T v) 
 template <class T> __device__ __forceinline__ T from_lane_below(T v) { return wave_shift_value<0x138>(v); }   // wave_shr:1
 template <class T> __device__ __forceinline__ T from_lane_above(T v) { return wave_shift_value<0x130>(v); }   // wave_shl:1
 
-#ifndef PU_X_F32_WAVES
-#define PU_X_F32_WAVES 8
-#endif
 template <int ORD, class T, int MODE>
 __global__ __launch_bounds__(SX_BX * SX_BY)
-__attribute__((amdgpu_waves_per_eu(std::is_same<T, float>::value ? PU_X_F32_WAVES : 1)))
+__attribute__((amdgpu_waves_per_eu(f64_waves(ORD))))
 void k_sweep_x(const T *__restrict__ prim, const uint16_t *__restrict__ codes, T *__restrict__ tend, SweepParams P,
                FuseArgs<T> FA) {
   constexpr int hs = (ORD - 1) / 2, hp = hs + 1;
@@ -700,7 +747,7 @@ void k_sweep_x(const T *__restrict__ prim, const uint16_t *__restrict__ codes, T
   // first stencil point of the cell below lane 0's
   const T *row = prim + ((long long)(k + hp) * P.nyh + (j + hp)) * P.nxh + (P.ox + c0 - hp);
   const unsigned lane = (unsigned)(t * (int)sizeof(T));
-  const long long crow = ((long long)k * P.ny + j) * P.nx, cid = crow + c;
+  const long long crow = ((long long)k * P.ny + j) * P.nx;
   // a periodic neighbour cell past either end is the wrapped interior cell
   unsigned own = 0;
   if (do_recon) own = codes[crow + (c < 0 ? c + n : (c >= n ? c - n : c))];
@@ -709,36 +756,34 @@ void k_sweep_x(const T *__restrict__ prim, const uint16_t *__restrict__ codes, T
 
   const T rd = (T)P.rd;
   const T hr = (T)P.hy_rc[hs + k], ht = (T)P.hy_tc[hs + k];
-  double f_rho = 0, f_u = 0, f_v = 0, f_mult = 0, f_trr = 0, f_trt = 0;
+  const long long cell0 = crow + c0;               // lane 0's cell
+  StageIn S{0., 0., 0., 0., 0., 0.};
   if constexpr (MODE == 2) {
-    if (has_tend) stage_inputs(FA, cid, k, f_rho, f_u, f_v, f_mult, f_trr, f_trt);
+    if (has_tend) S = stage_inputs(FA, cell0 + t, k);
   }
-  // FP64: the values a cell's finished tendency is combined with are loaded before the field's
-  // reconstruction, so their latency hides behind it.  FP32: loaded when needed -- the extra
-  // registers cost the FP32 kernel one wave of occupancy.
-  constexpr bool PREFETCH = std::is_same<T, double>::value;
+  // the values a cell's finished tendency is combined with are loaded before the field's
+  // reconstruction, so their latency hides behind it
   struct Pre { T t; double u, us; };
-  auto load_pre = [&](int fidx) {
+  auto prefetch = [&](int fidx) {
     Pre p{T(0), 0., 0.};
     if (has_tend) {
-      p.t = tend[(long long)fidx * P.n3 + cid];
+      p.t = load_at<T, unsigned>(tend + ((long long)fidx * P.n3 + cell0), lane);
       if constexpr (MODE == 2) {
-        p.u = load_cons(FA.U, FA.Ulo, fidx, cid, P.n3);
-        if (FA.C.stage > 0) p.us = load_cons(FA.Us, FA.Uslo, fidx, cid, P.n3);
+        p.u = load_cons_at(FA.U, fidx, cell0, lane, P.n3);
+        if (FA.C.stage > 0) p.us = load_cons_at(FA.Us, fidx, cell0, lane, P.n3);
       }
     }
     return p;
   };
-  auto prefetch = [&](int fidx) { return PREFETCH ? load_pre(fidx) : Pre{T(0), 0., 0.}; };
   // F: the flux through the cell's low face; completes the cell's tendency of one field
-  auto finish = [&](int fidx, T F, const Pre &pf0) {
+  auto finish = [&](int fidx, T F, const Pre &pf) {
     const T v = -(from_lane_above(F) - F) * rd;
     if (!has_tend) return;
-    const Pre pf = PREFETCH ? pf0 : load_pre(fidx);
     if constexpr (MODE == 2)
-      combine_field_v(FA, fidx, cid, (double)(pf.t + v), pf.u, pf.us, f_rho, f_u, f_v, f_mult, f_trr, f_trt);
+      store_at((FA.C.stage == 2 ? FA.U : FA.Us) + ((long long)fidx * P.n3 + cell0), lane,
+               combine_value(FA.C, fidx, pf.t + v, pf.u, pf.us, S));
     else
-      tend[(long long)fidx * P.n3 + cid] = pf.t + v;
+      store_at(tend + ((long long)fidx * P.n3 + cell0), lane, pf.t + v);
   };
 
   // ---- phase A: density, u, pressure -> acoustic upwinding ----
@@ -762,32 +807,28 @@ void k_sweep_x(const T *__restrict__ prim, const uint16_t *__restrict__ codes, T
     if (bface_hi) { rR = rL; uR = uL; pR = pL; }
     up = riemann(rL, uL, pL, rR, uR, pR, hr);
     Fr = up.ru;
-    Fu = up.ru * (up.left ? uL : uR) + up.p;
+    Fu = up.momentum(uL, uR);
   }
   finish(idR, Fr, preR);
   finish(idU, Fu, preU);
 
-  // ---- phase B: the transported quantities on the face's upwind side, one at a time ----
+  // ---- phase B: the transported quantities, one at a time ----
   // (the faces of an open boundary take the inner cell's value from either side)
   UpwindStencil<ORD, unsigned> us;
   us.setup(lane, (unsigned)sizeof(T), (up.left || bface_hi) && !bface_lo, lower, own);
   const bool weno_up = P.weno_all || (us.code & SC_ANY);
-  const int nB = 3 + P.ntr;
-  for (int b = 0; b < nB; b++) {
-    int l, fidx;
-    bool clamp;
-    transported<0>(b, l, fidx, clamp);
+  transport_all<0, true>(us, P.ntr, [&](bool theta, int l, int fidx, int) {
     const Pre pf = prefetch(fidx);
     T F = 0;
     if (has_face) {
       T s[ORD];
-      us.load(row + (long long)l * P.nh, clamp, s);
+      us.load(row + (long long)l * P.nh, s);
       T v = face_value<ORD, T>(s, us.code, weno_up);
-      if (l == idT) v += ht;
-      F = up.ru * v;
+      if (theta) v += ht;
+      F = carried(up.ru, v);
     }
     finish(fidx, F, pf);
-  }
+  });
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -870,7 +911,7 @@ __global__ __launch_bounds__(SG_BX * SG_BS) void k_sweep_seg(const T *__restrict
     if (wallz && (bface_lo || bface_hi)) { uL = 0; uR = 0; }     // W = 0 on both sides at walls
     up = riemann(rL, uL, pL, rR, uR, pR, hr);
     Fr = up.ru;
-    Fu = up.ru * (up.left ? uL : uR) + up.p;
+    Fu = up.momentum(uL, uR);
   }
   sA[0][lin] = Fr; sA[1][lin] = Fu;
   __syncthreads();
@@ -879,39 +920,41 @@ __global__ __launch_bounds__(SG_BX * SG_BS) void k_sweep_seg(const T *__restrict
     put(ln, -(sA[1][lin + BX] - Fu) * rd);
   }
 
-  // ---- phase B: the transported quantities on the face's upwind side, one at a time ----
-  UpwindStencil<ORD, long long> us;
-  us.setup(lane, stride, (up.left || bface_hi) && !bface_lo, lower, own);
-  const bool weno_up = P.weno_all || (us.code & SC_ANY);
-  const int nB = 3 + P.ntr;
-  for (int b = 0; b < nB; b++) {
-    int l, fidx;
-    bool clamp;
-    transported<DIR>(b, l, fidx, clamp);
-    T F = 0;
-    if (has_face) {
-      T s[ORD];
-      us.load(row + (long long)l * P.nh, clamp, s);
-      T v = face_value<ORD, T>(s, us.code, weno_up);
-      if (wallz && (bface_lo || bface_hi) && l == idT) v = 0;
-      if (l == idT) v += ht;
-      F = up.ru * v;
-    }
+  // ---- phase B: the transported quantities, one at a time ----
+  const bool left = (up.left || bface_hi) && !bface_lo;
+  const bool wall = wallz && (bface_lo || bface_hi);
+  auto through = [&](bool theta, T v) {
+    if (theta) v = (wall ? T(0) : v) + ht;
+    return carried(up.ru, v);
+  };
+  auto finish = [&](int fidx, int b, T F) {
     T *sF = sB[b & 1];
     sF[lin] = F;
     __syncthreads();
     if (has_tend) put(fidx, -(sF[lin + BX] - F) * rd);
-  }
+  };
+  UpwindStencil<ORD, long long> us;
+  us.setup(lane, stride, left, lower, own);
+  const bool weno_up = P.weno_all || (us.code & SC_ANY);
+  transport_all<DIR, false>(us, P.ntr, [&](bool theta, int l, int fidx, int b) {
+    T F = 0;
+    if (has_face) {
+      T s[ORD];
+      us.load(row + (long long)l * P.nh, s);
+      F = through(theta, face_value<ORD, T>(s, us.code, weno_up));
+    }
+    finish(fidx, b, F);
+  });
 }
 
-// FP32 whole-column z sweep (sweep_zwall_f32.hip)
+// FP32 (sweep_f32_core.h): whole-column z sweep (sweep_zwall_f32.hip), whole-line y sweep
+// (sweep_yline_f32.hip), segment sweeps (sweep_seg_f32.hip; dir 0: adds to the tendencies or, with
+// combine, finishes them through the stage combination; 1: adds; 2: writes)
 int launch_zwall_f32(int ord, dim3 grid, dim3 block, hipStream_t s, const float *prim, const uint16_t *codes,
                      float *tend, const SweepParams &P);
-// FP32 whole-line y sweep (sweep_yline_f32.hip)
 int launch_yline_f32(int ord, dim3 grid, dim3 block, hipStream_t s, const float *prim, const uint16_t *codes,
                      float *tend, const SweepParams &P);
-// FP32 x sweep (sweep_x_f32.hip), MODE 1 or 2
-int launch_x_f32(int ord, int mode, dim3 grid, dim3 block, hipStream_t s, const float *prim, const uint16_t *codes,
-                 float *tend, const SweepParams &P, const FuseArgs<float> &FA);
+int launch_seg_f32(int ord, int dir, bool combine, hipStream_t s, const float *prim, const uint16_t *codes, float *tend,
+                   const SweepParams &P, const FuseArgs<float> &FA);
 
 }  // namespace pu

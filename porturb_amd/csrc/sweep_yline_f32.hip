@@ -1,17 +1,17 @@
-// sweep_yline_f32.hip -- the FP32 whole-line y sweep (k_sweep_yline<ORD, float>, sweep_core.h) in a
+// sweep_yline_f32.hip -- the FP32 whole-line y sweep (f32::k_sweep_yline<ORD, float>, sweep_f32_core.h) in a
 // translation unit of its own, built with -mllvm -disable-machine-licm (porturb_amd/build.py).
-#include "sweep_core.h"
+#include "sweep_f32_core.h"
 
 namespace pu {
 
 int launch_yline_f32(int ord, dim3 grid, dim3 block, hipStream_t s, const float *prim, const uint16_t *codes,
                      float *tend, const SweepParams &P) {
   switch (ord) {
-    case 3: hipLaunchKernelGGL((k_sweep_yline<3, float>), grid, block, 0, s, prim, codes, tend, P); break;
-    case 5: hipLaunchKernelGGL((k_sweep_yline<5, float>), grid, block, 0, s, prim, codes, tend, P); break;
-    case 7: hipLaunchKernelGGL((k_sweep_yline<7, float>), grid, block, 0, s, prim, codes, tend, P); break;
-    case 9: hipLaunchKernelGGL((k_sweep_yline<9, float>), grid, block, 0, s, prim, codes, tend, P); break;
-    case 11: hipLaunchKernelGGL((k_sweep_yline<11, float>), grid, block, 0, s, prim, codes, tend, P); break;
+    case 3: hipLaunchKernelGGL((f32::k_sweep_yline<3, float>), grid, block, 0, s, prim, codes, tend, P); break;
+    case 5: hipLaunchKernelGGL((f32::k_sweep_yline<5, float>), grid, block, 0, s, prim, codes, tend, P); break;
+    case 7: hipLaunchKernelGGL((f32::k_sweep_yline<7, float>), grid, block, 0, s, prim, codes, tend, P); break;
+    case 9: hipLaunchKernelGGL((f32::k_sweep_yline<9, float>), grid, block, 0, s, prim, codes, tend, P); break;
+    case 11: hipLaunchKernelGGL((f32::k_sweep_yline<11, float>), grid, block, 0, s, prim, codes, tend, P); break;
     default: return fail(PU_ERR_UNSUPPORTED, "unsupported ord");
   }
   PU_HIP_CHECK(hipGetLastError());

@@ -69,10 +69,11 @@ def recon_flops_flat(ord_, sides="LR"):
     return _tv_flops(ord_) + linear_flops(ord_, sides)
 
 
-def per_field(nf, flops):
+def per_field(nf, flops, upwind):
     """Average over a sweep's nf fields of flops(sides): density, normal velocity and pressure are
-    reconstructed on both sides of a cell, the transported quantities on a face's upwind side."""
-    return (3 * flops("LR") + (nf - 3) * flops("R")) / nf
+    reconstructed on both sides of a cell, the transported quantities on a face's upwind side
+    (`upwind`: the FP64 sweeps) or on both."""
+    return (3 * flops("LR") + (nf - 3) * flops("R" if upwind else "LR")) / nf
 
 
 def sweep_overhead_flops(nf):
@@ -84,21 +85,22 @@ def sweep_overhead_flops(nf):
     return riemann + advected + divergence
 
 
-def executed_sweep_flops(ord_, nf, census_row, cells):
+def executed_sweep_flops(ord_, nf, census_row, cells, upwind=True):
     """FLOPs one sweep launch executes over `cells` cells, from the reconstruction census of the
     state (counts of the limiter, flat-stencil and linear branches over all fields, so each branch
     is priced at its average over the fields)."""
     n_lim, n_flat, n_lin = (int(v) for v in census_row)
-    return (n_lim * per_field(nf, lambda sides: recon_flops(ord_, sides=sides))
-            + n_flat * per_field(nf, lambda sides: recon_flops_flat(ord_, sides))
-            + n_lin * per_field(nf, lambda sides: linear_flops(ord_, sides)) + cells * sweep_overhead_flops(nf))
+    return (n_lim * per_field(nf, lambda sides: recon_flops(ord_, sides=sides), upwind)
+            + n_flat * per_field(nf, lambda sides: recon_flops_flat(ord_, sides), upwind)
+            + n_lin * per_field(nf, lambda sides: linear_flops(ord_, sides), upwind)
+            + cells * sweep_overhead_flops(nf))
 
 
-def sweep_flops_per_cell(ord_, nf):
-    """One direction: nf reconstructions (three on both sides, the others on the upwind side), the
+def sweep_flops_per_cell(ord_, nf, upwind=True):
+    """One direction: nf reconstructions (see per_field), the
     acoustic Riemann solve at one face, upwinded fluxes and the flux divergence of nf-1 conserved
     variables."""
-    return nf * per_field(nf, lambda sides: recon_flops(ord_, sides=sides)) + sweep_overhead_flops(nf)
+    return nf * per_field(nf, lambda sides: recon_flops(ord_, sides=sides), upwind) + sweep_overhead_flops(nf)
 
 
 def step_flops_per_cell(ord_, nf):
