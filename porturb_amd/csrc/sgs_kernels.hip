@@ -116,19 +116,37 @@ struct TrainArgs {
   float scale;          // 2 / (n * NOUT)
 };
 
+// LDS of one training block (shorts).  A layer's result sits in the lanes as the next layer's operand
+// needs it (unit 4g + r, sample r16), so activations stay in registers; only the weight gradients, whose
+// K is the samples, read them by unit, from the transposed copies XT ... DYT.  Rows are padded to an odd
+// number of 8-byte words so that the 16 lanes of a fragment read different banks, and every matrix
+// operand is one 8-byte read.
+constexpr int LDX = NINP + 4, LDH = NH + 4, LDO = NOUTP + 4, LDT = SAMPLES_PER_BLOCK + 4;
+struct TrainLds {
+  static constexpr int X = 0, W1 = X + SAMPLES_PER_BLOCK * LDX, W2 = W1 + NH * LDX, W3 = W2 + NH * LDH,
+                       FORWARD = W3 + NOUTP * LDH, W2T = FORWARD, W3T = W2T + NH * LDH, XT = W3T + NH * LDO,
+                       A1T = XT + NINP * LDT, A2T = A1T + NH * LDT, D1T = A2T + NH * LDT, D2T = D1T + NH * LDT,
+                       DYT = D2T + NH * LDT, ALL = DYT + NOUTP * LDT;
+  static constexpr size_t bytes(bool train) { return 2 * (size_t)(train ? ALL : FORWARD); }
+};
+
+// 64 samples per block, one 16-sample tile per wave.  A batch of 8192 is 128 blocks, less than one per
+// CU: what bounds it is the latency of the chain input gather -> three layers -> backward -> weight
+// gradients of a single block, not any rate.  17.3 us for 8192 samples (23.5 under the same
+// profile with the weights read from memory inside the layer loops and the transposed operands gathered
+// by 2-byte reads); the forward pass over 4 million samples takes 335 us (992), 2.7 TB/s of inputs.
 template <bool TRAIN>
 __global__ __launch_bounds__(256) void k_mlp_train(TrainArgs A) {
-  __shared__ __align__(16) short sX[SAMPLES_PER_BLOCK * NINP];
-  __shared__ __align__(16) short sA1[SAMPLES_PER_BLOCK * NH], sA2[SAMPLES_PER_BLOCK * NH];
-  __shared__ __align__(16) short sD1[SAMPLES_PER_BLOCK * NH], sD2[SAMPLES_PER_BLOCK * NH];
-  __shared__ __align__(16) short sDY[SAMPLES_PER_BLOCK * NOUTP];
+  extern __shared__ __align__(16) short sm[];
   __shared__ float sBias[4][NH + NH + NOUTP];
   __shared__ float sLoss[4];
+  using L = TrainLds;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r16 = lane & 15, g = lane >> 4;
   const long long base = (long long)blockIdx.x * SAMPLES_PER_BLOCK;
-  // stage the block's inputs (rows beyond n are zero); all loads issued before the LDS writes
-  constexpr int PER = SAMPLES_PER_BLOCK * (NINP / 4) / 256;
-  uint2 xin[PER];
+  // stage the block's inputs (rows beyond n are zero) and the weights; all loads issued before the
+  // LDS writes
+  constexpr int PER = SAMPLES_PER_BLOCK * (NINP / 4) / 256, PW1 = NH * (NINP / 4) / 256, PW2 = NH * (NH / 4) / 256;
+  uint2 xin[PER], w1[PW1], w2[PW2];
 #pragma unroll
   for (int e = 0; e < PER; e++) {
     const int c = tid + 256 * e;
@@ -141,67 +159,113 @@ __global__ __launch_bounds__(256) void k_mlp_train(TrainArgs A) {
     }
   }
 #pragma unroll
+  for (int e = 0; e < PW1; e++) w1[e] = reinterpret_cast<const uint2 *>(A.wbf + P_W1)[tid + 256 * e];
+#pragma unroll
+  for (int e = 0; e < PW2; e++) w2[e] = reinterpret_cast<const uint2 *>(A.wbf + P_W2)[tid + 256 * e];
+  const uint2 w3 = reinterpret_cast<const uint2 *>(A.wbf + P_W3)[tid];      // NOUTP * NH / 4 = 256
+  auto put8 = [&](short *dst, uint2 v) { *reinterpret_cast<uint2 *>(dst) = v; };
+  auto put_t = [&](int dst, int ld, int row, int col, uint2 v) {      // transposed: element (row, col + i) to [col + i][row]
+    const short e[4] = {(short)v.x, (short)(v.x >> 16), (short)v.y, (short)(v.y >> 16)};
+#pragma unroll
+    for (int i = 0; i < 4; i++) sm[dst + (col + i) * ld + row] = e[i];
+  };
+#pragma unroll
+  for (int e = 0; e < PW1; e++) {
+    const int c = tid + 256 * e;
+    put8(sm + L::W1 + (c / (NINP / 4)) * LDX + 4 * (c % (NINP / 4)), w1[e]);
+  }
+#pragma unroll
+  for (int e = 0; e < PW2; e++) {
+    const int c = tid + 256 * e;
+    put8(sm + L::W2 + (c / (NH / 4)) * LDH + 4 * (c % (NH / 4)), w2[e]);
+    if (TRAIN) put_t(L::W2T, LDH, c / (NH / 4), 4 * (c % (NH / 4)), w2[e]);
+  }
+  put8(sm + L::W3 + (tid / (NH / 4)) * LDH + 4 * (tid % (NH / 4)), w3);
+  if (TRAIN) put_t(L::W3T, LDO, tid / (NH / 4), 4 * (tid % (NH / 4)), w3);
+#pragma unroll
   for (int e = 0; e < PER; e++) {
     const int c = tid + 256 * e;
-    *reinterpret_cast<uint2 *>(sX + (c / (NINP / 4)) * NINP + 4 * (c % (NINP / 4))) = xin[e];
+    put8(sm + L::X + (c / (NINP / 4)) * LDX + 4 * (c % (NINP / 4)), xin[e]);
+    if (TRAIN) put_t(L::XT, LDT, c / (NINP / 4), 4 * (c % (NINP / 4)), xin[e]);
   }
-  __syncthreads();
   const int my = 16 * w + r16;                    // this lane's sample column within the block
   const long long gsample = base + my;
   const bool valid = gsample < A.n;
   const long long row = valid ? (A.idx ? (long long)A.idx[gsample] : gsample) : 0;
+  float tgt[4] = {0.f, 0.f, 0.f, 0.f};
+  if (TRAIN && valid) {
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+      if (4 * g + r < NOUT) tgt[r] = A.T[row * NOUT + 4 * g + r];
+  }
+  fx4 b1[4], b2[4];
+#pragma unroll
+  for (int mt = 0; mt < 4; mt++) {
+    b1[mt] = *reinterpret_cast<const fx4 *>(A.master + P_B1 + 16 * mt + 4 * g);
+    b2[mt] = *reinterpret_cast<const fx4 *>(A.master + P_B2 + 16 * mt + 4 * g);
+  }
+  const fx4 b3 = *reinterpret_cast<const fx4 *>(A.master + P_B3 + 4 * g);
+  __syncthreads();
 
   // ---- forward ----
-  float h1[4][4], h2[4][4];
+  fx4 h1[4], h2[4];
+  bfx4 a1[4], a2[4];
+#pragma unroll
   for (int mt = 0; mt < 4; mt++) {
     fx4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
     for (int kb = 0; kb < NINP / 16; kb++)
-      acc = mfma16(ld4(A.wbf + P_W1 + (16 * mt + r16) * NINP + 16 * kb + 4 * g), ld4(sX + my * NINP + 16 * kb + 4 * g), acc);
+      acc = mfma16(ld4(sm + L::W1 + (16 * mt + r16) * LDX + 16 * kb + 4 * g), ld4(sm + L::X + my * LDX + 16 * kb + 4 * g), acc);
+#pragma unroll
     for (int r = 0; r < 4; r++) {
-      const int u = 16 * mt + 4 * g + r;
-      const float h = acc[r] + A.master[P_B1 + u];
-      h1[mt][r] = h;
-      sA1[my * NH + u] = bf16_bits(relu(h));
+      h1[mt][r] = acc[r] + b1[mt][r];
+      a1[mt][r] = bf16_bits(relu(h1[mt][r]));
+      if (TRAIN) sm[L::A1T + (16 * mt + 4 * g + r) * LDT + my] = a1[mt][r];
     }
   }
-  __syncthreads();
+#pragma unroll
   for (int mt = 0; mt < 4; mt++) {
     fx4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
     for (int kb = 0; kb < NH / 16; kb++)
-      acc = mfma16(ld4(A.wbf + P_W2 + (16 * mt + r16) * NH + 16 * kb + 4 * g), ld4(sA1 + my * NH + 16 * kb + 4 * g), acc);
+      acc = mfma16(ld4(sm + L::W2 + (16 * mt + r16) * LDH + 16 * kb + 4 * g), a1[kb], acc);
+#pragma unroll
     for (int r = 0; r < 4; r++) {
-      const int u = 16 * mt + 4 * g + r;
-      const float h = acc[r] + A.master[P_B2 + u];
-      h2[mt][r] = h;
-      sA2[my * NH + u] = bf16_bits(relu(h));
+      h2[mt][r] = acc[r] + b2[mt][r];
+      a2[mt][r] = bf16_bits(relu(h2[mt][r]));
+      if (TRAIN) sm[L::A2T + (16 * mt + 4 * g + r) * LDT + my] = a2[mt][r];
     }
   }
-  __syncthreads();
   fx4 yacc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
   for (int kb = 0; kb < NH / 16; kb++)
-    yacc = mfma16(ld4(A.wbf + P_W3 + r16 * NH + 16 * kb + 4 * g), ld4(sA2 + my * NH + 16 * kb + 4 * g), yacc);
+    yacc = mfma16(ld4(sm + L::W3 + r16 * LDH + 16 * kb + 4 * g), a2[kb], yacc);
   // lane holds output o = 4g + r of sample `my`
   if (!TRAIN) {
     for (int r = 0; r < 4; r++) {
       const int o = 4 * g + r;
-      if (o < NOUT && valid) A.Y[gsample * NOUT + o] = yacc[r] + A.master[P_B3 + o];
+      if (o < NOUT && valid) A.Y[gsample * NOUT + o] = yacc[r] + b3[r];
     }
     return;
   }
 
   // ---- backward ----
   float lossp = 0.f, dyv[4];
+  bfx4 dyb;
+#pragma unroll
   for (int r = 0; r < 4; r++) {
     const int o = 4 * g + r;
     float d = 0.f;
     if (o < NOUT && valid) {
-      const float e = (yacc[r] + A.master[P_B3 + o]) - A.T[row * NOUT + o];
+      const float e = (yacc[r] + b3[r]) - tgt[r];
       lossp += e * e;
       d = A.scale * e;
     }
     dyv[r] = d;
-    sDY[my * NOUTP + o] = bf16_bits(d);
+    dyb[r] = bf16_bits(d);
+    sm[L::DYT + o * LDT + my] = dyb[r];
   }
+#pragma unroll
   for (int r = 0; r < 4; r++) {
     const float v = sum16(dyv[r]);
     if (r16 == 0) sBias[w][2 * NH + 4 * g + r] = v;
@@ -212,34 +276,34 @@ __global__ __launch_bounds__(256) void k_mlp_train(TrainArgs A) {
     v += __shfl_xor(v, 32);
     if (lane == 0) sLoss[w] = v;
   }
-  __syncthreads();
   // dA2 = W3^T dy, dH2 = dA2 * relu'(h2)
+  bfx4 d2[4];
+#pragma unroll
   for (int mt = 0; mt < 4; mt++) {
-    bfx4 a;
-    for (int q = 0; q < 4; q++) a[q] = A.wbf[P_W3 + (4 * g + q) * NH + 16 * mt + r16];
     fx4 acc = {0.f, 0.f, 0.f, 0.f};
-    acc = mfma16(a, ld4(sDY + my * NOUTP + 4 * g), acc);
+    acc = mfma16(ld4(sm + L::W3T + (16 * mt + r16) * LDO + 4 * g), dyb, acc);
+#pragma unroll
     for (int r = 0; r < 4; r++) {
       const int u = 16 * mt + 4 * g + r;
       const float d = acc[r] * relu_deriv(h2[mt][r]);
-      sD2[my * NH + u] = bf16_bits(d);
+      d2[mt][r] = bf16_bits(d);
+      sm[L::D2T + u * LDT + my] = d2[mt][r];
       const float v = sum16(d);
       if (r16 == 0) sBias[w][NH + u] = v;
     }
   }
-  __syncthreads();
   // dA1 = W2^T dH2, dH1 = dA1 * relu'(h1)
+#pragma unroll
   for (int mt = 0; mt < 4; mt++) {
     fx4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int kb = 0; kb < NH / 16; kb++) {
-      bfx4 a;
-      for (int q = 0; q < 4; q++) a[q] = A.wbf[P_W2 + (16 * kb + 4 * g + q) * NH + 16 * mt + r16];
-      acc = mfma16(a, ld4(sD2 + my * NH + 16 * kb + 4 * g), acc);
-    }
+#pragma unroll
+    for (int kb = 0; kb < NH / 16; kb++)
+      acc = mfma16(ld4(sm + L::W2T + (16 * mt + r16) * LDH + 16 * kb + 4 * g), d2[kb], acc);
+#pragma unroll
     for (int r = 0; r < 4; r++) {
       const int u = 16 * mt + 4 * g + r;
       const float d = acc[r] * relu_deriv(h1[mt][r]);
-      sD1[my * NH + u] = bf16_bits(d);
+      sm[L::D1T + u * LDT + my] = bf16_bits(d);
       const float v = sum16(d);
       if (r16 == 0) sBias[w][u] = v;
     }
@@ -247,22 +311,19 @@ __global__ __launch_bounds__(256) void k_mlp_train(TrainArgs A) {
   __syncthreads();
   // weight gradients, K = the block's 64 samples: dW[out][in] = sum_s dH[s][out] * act[s][in]
   float *out = A.partial + (size_t)blockIdx.x * P_N;
-  auto wgrad = [&](const short *dH, int ldh, int mt, const short *act, int lda, int nt, float *dst, int ldd) {
+  auto wgrad = [&](int dH, int mt, int act, int nt, float *dst, int ldd) {
     fx4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int kb = 0; kb < SAMPLES_PER_BLOCK / 16; kb++) {
-      bfx4 a, b;
-      for (int q = 0; q < 4; q++) {
-        const int s = 16 * kb + 4 * g + q;
-        a[q] = dH[s * ldh + 16 * mt + r16];
-        b[q] = act[s * lda + 16 * nt + r16];
-      }
-      acc = mfma16(a, b, acc);
-    }
+#pragma unroll
+    for (int kb = 0; kb < SAMPLES_PER_BLOCK / 16; kb++)
+      acc = mfma16(ld4(sm + dH + (16 * mt + r16) * LDT + 16 * kb + 4 * g), ld4(sm + act + (16 * nt + r16) * LDT + 16 * kb + 4 * g), acc);
+#pragma unroll
     for (int r = 0; r < 4; r++) dst[(16 * mt + 4 * g + r) * ldd + 16 * nt + r16] = acc[r];
   };
-  wgrad(sDY, NOUTP, 0, sA2, NH, w, out + P_W3, NH);                           // dW3: 4 tiles, one per wave
-  for (int nt = 0; nt < 4; nt++) wgrad(sD2, NH, w, sA1, NH, nt, out + P_W2, NH);       // dW2: 16 tiles
-  for (int nt = 0; nt < NINP / 16; nt++) wgrad(sD1, NH, w, sX, NINP, nt, out + P_W1, NINP);  // dW1: 28 tiles
+  wgrad(L::DYT, 0, L::A2T, w, out + P_W3, NH);                               // dW3: 4 tiles, one per wave
+#pragma unroll
+  for (int nt = 0; nt < 4; nt++) wgrad(L::D2T, w, L::A1T, nt, out + P_W2, NH);          // dW2: 16 tiles
+#pragma unroll
+  for (int nt = 0; nt < NINP / 16; nt++) wgrad(L::D1T, w, L::XT, nt, out + P_W1, NINP);   // dW1: 28 tiles
   for (int u = tid; u < NH + NH + NOUTP; u += 256) {
     const float v = sBias[0][u] + sBias[1][u] + sBias[2][u] + sBias[3][u];
     const int dst = u < NH ? P_B1 + u : (u < 2 * NH ? P_B2 + (u - NH) : P_B3 + (u - 2 * NH));
@@ -283,14 +344,24 @@ struct ReduceArgs {
   float lr, b1, b2, eps, c1, c2;
 };
 
-__global__ __launch_bounds__(256) void k_mlp_reduce(ReduceArgs A) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
+// One thread per parameter sums the blocks in order; RED_BATCH of their values are loaded ahead of the
+// additions and 64-thread blocks spread the 12432 parameters over 195 CUs instead of 49:
+// 6.2 us for 128 blocks, 31 us with one load per addition in 256-thread blocks.  Same order, same bits.
+constexpr int RED_THREADS = 64, RED_BATCH = 32;
+__global__ __launch_bounds__(RED_THREADS) void k_mlp_reduce(ReduceArgs A) {
+  const int p = blockIdx.x * RED_THREADS + threadIdx.x;
   if (p >= P_N) return;
   float gsum;
   if (A.gin) gsum = A.gin[p];
   else {
     gsum = 0.f;
-    for (int b = 0; b < A.nblocks; b++) gsum += A.partial[(size_t)b * P_N + p];
+    for (int b0 = 0; b0 < A.nblocks; b0 += RED_BATCH) {
+      float v[RED_BATCH];
+#pragma unroll
+      for (int i = 0; i < RED_BATCH; i++) v[i] = b0 + i < A.nblocks ? A.partial[(size_t)(b0 + i) * P_N + p] : 0.f;
+#pragma unroll
+      for (int i = 0; i < RED_BATCH; i++) gsum += v[i];
+    }
   }
   if (A.grad) A.grad[p] = gsum;
   if (!A.update) return;
@@ -694,7 +765,9 @@ static int mlp_batch(pu_mlp *m, const short *Xbf, const float *T, const int *idx
   int rc = mlp_ensure_blocks(m, nb);
   if (rc) return rc;
   TrainArgs A{Xbf, T, idx, n, m->d_wbf, m->d_master, m->d_partial, m->d_ploss, nullptr, 2.f / ((float)n * NOUT)};
-  hipLaunchKernelGGL(k_mlp_train<true>, dim3(nb), dim3(256), 0, 0, A);
+  constexpr size_t lds = TrainLds::bytes(true);
+  PU_HIP_CHECK(hipFuncSetAttribute((const void *)k_mlp_train<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  hipLaunchKernelGGL(k_mlp_train<true>, dim3(nb), dim3(256), lds, 0, A);
   PU_HIP_CHECK(hipGetLastError());
   if (loss) {
     std::vector<float> pl(nb);
@@ -717,7 +790,7 @@ static int mlp_reduce(pu_mlp *m, int nblocks, const float *gin, float *grad_out,
     R.c1 = 1.f - powf(R.b1, (float)m->t);
     R.c2 = 1.f - powf(R.b2, (float)m->t);
   }
-  hipLaunchKernelGGL(k_mlp_reduce, dim3((P_N + 255) / 256), dim3(256), 0, 0, R);
+  hipLaunchKernelGGL(k_mlp_reduce, dim3((P_N + RED_THREADS - 1) / RED_THREADS), dim3(RED_THREADS), 0, 0, R);
   PU_HIP_CHECK(hipGetLastError());
   return PU_OK;
 }
@@ -906,7 +979,8 @@ int pu_mlp_forward(pu_mlp *m, const unsigned short *Xbf, const int *idx, int n, 
   if (!m || !Xbf || !Y || n <= 0) return fail(PU_ERR_ARG, "pu_mlp_forward: null argument or n <= 0");
   const int nb = (n + SAMPLES_PER_BLOCK - 1) / SAMPLES_PER_BLOCK;
   TrainArgs A{(const short *)Xbf, nullptr, idx, n, m->d_wbf, m->d_master, nullptr, nullptr, Y, 0.f};
-  hipLaunchKernelGGL(k_mlp_train<false>, dim3(nb), dim3(256), 0, 0, A);
+  constexpr size_t lds = TrainLds::bytes(false);
+  hipLaunchKernelGGL(k_mlp_train<false>, dim3(nb), dim3(256), lds, 0, A);
   PU_HIP_CHECK(hipGetLastError());
   PU_HIP_CHECK(hipDeviceSynchronize());
   return PU_OK;
