@@ -75,15 +75,15 @@ __global__ __launch_bounds__(256) void k_les_prim(const double *__restrict__ rd_
   vals[1] = uu[sid];
   vals[2] = vv[sid];
   vals[3] = ww[sid];
-  vals[4] = pow(rho_d * P.R_d * tt[sid] / P.C0, 1. / P.gamma) / rho_d;
+  vals[4] = pow_pos(rho_d * P.R_d * tt[sid] / P.C0, 1. / P.gamma) / rho_d;
   vals[5] = fmax(0., trc.p[P.idTKE][sid] / rho_d);
   if (zhalo && P.bc_z != PU_BC_PERIODIC) {
     vals[3] = 0.;
     // hydrostatic extrapolation of rho from the first interior level (les_closure.h:503-510)
     double g = P.enable_gravity ? P.grav : 0.;
-    double rho0_gm1 = pow(rho_d, P.gamma - 1), theta0_g = pow(vals[4], P.gamma);
+    double rho0_gm1 = pow_pos(rho_d, P.gamma - 1), theta0_g = pow_pos(vals[4], P.gamma);
     double sgn = k < 0 ? 1. : -1.;
-    vals[0] = pow(rho0_gm1 + sgn * g * (P.gamma - 1) * P.dz * 1 / (P.gamma * P.C0 * theta0_g), 1. / (P.gamma - 1));
+    vals[0] = pow_pos(rho0_gm1 + sgn * g * (P.gamma - 1) * P.dz * 1 / (P.gamma * P.C0 * theta0_g), 1. / (P.gamma - 1));
   }
   for (int f = 0; f < 6; f++) F[(long long)f * P.nh + id] = (T)vals[f];
   for (int q = 0; q < P.nq; q++) F[(long long)(6 + q) * P.nh + id] = (T)(trc.p[P.qidx[q]][sid] / rho_d);
@@ -463,7 +463,7 @@ __global__ __launch_bounds__(LES_THREADS) void k_les_update(const T *__restrict_
     uu[id] = ru * rrho;
     vv[id] = rv * rrho;
     ww[id] = rw * rrho;
-    tt[id] = P.C0 * pow(rt, P.gamma) * (rrho * P.rR_d);
+    tt[id] = P.C0 * pow_pos(rt, P.gamma) * (rrho * P.rR_d);
     trc.p[P.idTKE][id] = rk;
   } else {
     uu[id] += (double)(dt * tend[0] * rrho);

@@ -411,7 +411,7 @@ __global__ __launch_bounds__(256) void k_sgs_filter(FilterArgs A) {
       for (int e = 0; e < A.r; e++) {
         const long long f = ((long long)(K * A.r + a) * A.ny + (J * A.r + b)) * A.nx + (I * A.r + e);
         const double rho = A.rho[f], u = A.u[f], v = A.v[f], w = A.w[f];
-        const double th = pow(rho * A.R_d * A.T[f] / A.C0, A.inv_gamma) / rho;
+        const double th = pow_pos(rho * A.R_d * A.T[f] / A.C0, A.inv_gamma) / rho;
         m[0] += rho; m[1] += u; m[2] += v; m[3] += w; m[4] += th;
         uu[0] += u * u; uu[1] += u * v; uu[2] += u * w; uu[3] += v * v; uu[4] += v * w; uu[5] += w * w;
         ut[0] += u * th; ut[1] += v * th; ut[2] += w * th;
