@@ -94,7 +94,7 @@ int pu_create(const pu_config *cfg, void *stream, pu_ctx **out) {
   if (hipGetDevice(&c->device) != hipSuccess) { delete c; return fail(PU_ERR_HIP, "hipGetDevice failed"); }
   if (getenv("PORTURB_SEGMENT_SWEEPS")) {
     const char *dirs = getenv("PORTURB_SEGMENT_DIRS");      // optional subset, e.g. "z" or "xy"
-    for (int d = 0; d < 3; d++) c->segment_sweeps[d] = !dirs || strchr(dirs, "xyz"[d]) != nullptr;
+    for (int d = 0; d < 3; d++) c->sweep_route[d] = !dirs || strchr(dirs, "xyz"[d]) ? pu_ctx::ROUTE_SEGMENTS : pu_ctx::ROUTE_LINES;
   }
   Grid &g = c->g;
   g.nx = cfg->nx; g.ny = cfg->ny; g.nz = cfg->nz;

@@ -338,8 +338,29 @@ static SweepParams sweep_params(pu_ctx *ctx, int dir) {
   return P;
 }
 
-// z sweep: writes d_tend.  Between solid walls the whole-column kernel, otherwise (periodic z, or
-// columns whose offsets need more than 32 bits) the segment kernel.
+// Whole lines (blocks that walk CH_BX lines in chunks of CH_BS cells) or segments (blocks of SG_NC cells and
+// a neighbour at each end)?  A line's rounds are its chunks; the last round of blocks is part empty, which
+// costs about slots / blocks of a round; a segment's thread costs `rel` of a chunk's, less where the
+// order is low and the line's carries weigh more.  us per launch, lines then segments:
+//   y FP64       512x512x128 order 5: 2715, 2108   order 9: 3679, 3925     500x310x90 order 5: 1242, 889
+//                96x200x33   order 9: 142, 83      64x64x64 order 5: 43, 30
+//   z FP64/FP32  512x512x128 order 5: 2268, 2573 / 1558, 1687   order 9: 3543, 4381 / 2342, 2834
+//                500x310x90  order 5: 959, 870 / 675, 593       order 9: 1494, 1477 / 1002, 976
+//                150x70x51   order 7: 74, 60 / 55, 51           16x16x128 order 9: 74, 23 / 70, 22
+// In FP32 the y lines always take the line kernel: the two round differently there, and the limiter's map
+// would carry that into single cells (see sweep_f32_core.h).
+template <int ORD, class T> static bool by_segments(const pu_ctx *ctx, int dir, long long blocks, int cells) {
+  if (ctx->sweep_route[dir] != pu_ctx::ROUTE_RULE) return ctx->sweep_route[dir] == pu_ctx::ROUTE_SEGMENTS;
+  constexpr bool f32 = std::is_same<T, float>::value;
+  if (f32 && dir == 1) return false;
+  const double rel = ORD < 9 ? (dir == 1 ? 0.77 : 0.9) : dir == 1 ? 0.96 : f32 ? 1. : 1.03;
+  const double slots = dir == 1 ? 320. : 240.;
+  const int chunks = (cells + CH_BS - 1) / CH_BS, segments = (cells + SG_NC - 1) / SG_NC;
+  return rel * segments < chunks * (1. + slots / (double)blocks);
+}
+
+// z sweep: writes d_tend.  Between solid walls by whole columns or segments (by_segments), otherwise
+// (periodic z, or columns whose offsets need more than 32 bits) by segments.
 template <int ORD, class T>
 static int sweep_z(pu_ctx *ctx, hipStream_t s) {
   const pu::Grid &g = ctx->g;
@@ -348,22 +369,22 @@ static int sweep_z(pu_ctx *ctx, hipStream_t s) {
   const T *prim = (const T *)ctx->d_prim;
   T *tend = (T *)ctx->d_tend;
   const uint16_t *codes = ctx->d_codes + 2 * g.n3();
-  if (!ctx->segment_sweeps[2] && P.wall_z && offsets_fit<T>(g.nxh * g.nyh, g.hp)) {
-    const dim3 blk(CH_BX, CH_BS, 1), grd((unsigned)((g.nx + CH_BX - 1) / CH_BX), (unsigned)g.ny, 1);
+  const dim3 blk(CH_BX, CH_BS, 1), grd((unsigned)((g.nx + CH_BX - 1) / CH_BX), (unsigned)g.ny, 1);
+  if (P.wall_z && offsets_fit<T>(g.nxh * g.nyh, g.hp) && !by_segments<ORD, T>(ctx, 2, (long long)grd.x * grd.y, g.nz)) {
     if constexpr (std::is_same<T, float>::value) return launch_zwall_f32(ORD, grd, blk, s, prim, codes, tend, P);
     else hipLaunchKernelGGL((k_sweep_zwall<ORD, T>), grd, blk, 0, s, prim, codes, tend, P);
   } else if constexpr (std::is_same<T, float>::value) {
     return launch_seg_f32(ORD, 2, false, s, prim, codes, tend, P, FuseArgs<float>{});
   } else {
-    const dim3 blk(SG_BX, SG_BS, 1);
-    const dim3 grd((unsigned)((g.nx + SG_BX - 1) / SG_BX), (unsigned)g.ny, (unsigned)((g.nz + SG_NC - 1) / SG_NC));
-    hipLaunchKernelGGL((k_sweep_seg<ORD, T, 2>), grd, blk, 0, s, prim, codes, tend, P);
+    const dim3 sblk(SG_BX, SG_BS, 1);
+    const dim3 sgrd((unsigned)((g.nx + SG_BX - 1) / SG_BX), (unsigned)g.ny, (unsigned)((g.nz + SG_NC - 1) / SG_NC));
+    hipLaunchKernelGGL((k_sweep_seg<ORD, T, 2>), sgrd, sblk, 0, s, prim, codes, tend, P);
   }
   PU_HIP_CHECK(hipGetLastError());
   return PU_OK;
 }
 
-// y sweep: adds to d_tend.  Periodic lines the whole-line kernel, otherwise the segment kernel.
+// y sweep: adds to d_tend.  Periodic lines by whole lines or segments (by_segments), otherwise segments.
 template <int ORD, class T>
 static int sweep_y(pu_ctx *ctx, hipStream_t s) {
   const pu::Grid &g = ctx->g;
@@ -372,16 +393,17 @@ static int sweep_y(pu_ctx *ctx, hipStream_t s) {
   const T *prim = (const T *)ctx->d_prim;
   T *tend = (T *)ctx->d_tend;
   const uint16_t *codes = ctx->d_codes + g.n3();
-  if (!ctx->segment_sweeps[1] && P.bc_along == PU_BC_PERIODIC && offsets_fit<T>(g.nxh, g.hp)) {
-    const dim3 blk(CH_BX, CH_BS, 1), grd((unsigned)((g.nx + CH_BX - 1) / CH_BX), (unsigned)g.nz, 1);
+  const dim3 blk(CH_BX, CH_BS, 1), grd((unsigned)((g.nx + CH_BX - 1) / CH_BX), (unsigned)g.nz, 1);
+  if (P.bc_along == PU_BC_PERIODIC && offsets_fit<T>(g.nxh, g.hp) &&
+      !by_segments<ORD, T>(ctx, 1, (long long)grd.x * grd.y, g.ny)) {
     if constexpr (std::is_same<T, float>::value) return launch_yline_f32(ORD, grd, blk, s, prim, codes, tend, P);
     else hipLaunchKernelGGL((k_sweep_yline<ORD, T>), grd, blk, 0, s, prim, codes, tend, P);
   } else if constexpr (std::is_same<T, float>::value) {
     return launch_seg_f32(ORD, 1, false, s, prim, codes, tend, P, FuseArgs<float>{});
   } else {
-    const dim3 blk(SG_BX, SG_BS, 1);
-    const dim3 grd((unsigned)((g.nx + SG_BX - 1) / SG_BX), (unsigned)((g.ny + SG_NC - 1) / SG_NC), (unsigned)g.nz);
-    hipLaunchKernelGGL((k_sweep_seg<ORD, T, 1>), grd, blk, 0, s, prim, codes, tend, P);
+    const dim3 sblk(SG_BX, SG_BS, 1);
+    const dim3 sgrd((unsigned)((g.nx + SG_BX - 1) / SG_BX), (unsigned)((g.ny + SG_NC - 1) / SG_NC), (unsigned)g.nz);
+    hipLaunchKernelGGL((k_sweep_seg<ORD, T, 1>), sgrd, sblk, 0, s, prim, codes, tend, P);
   }
   PU_HIP_CHECK(hipGetLastError());
   return PU_OK;

@@ -54,7 +54,9 @@ struct pu_ctx {
   bool les_ready = false;
   // sweeps through the segment kernel (environment variable PORTURB_SEGMENT_SWEEPS set when the
   // context is created): the whole-line kernels are checked against it
-  bool segment_sweeps[3] = {false, false, false};   // x, y, z (PORTURB_SEGMENT_DIRS narrows it)
+  // y and z sweeps: by the rule of by_segments, or (PORTURB_SEGMENT_SWEEPS) segments in the directions of
+  // PORTURB_SEGMENT_DIRS and whole lines in the others
+  enum SweepRoute { ROUTE_RULE, ROUTE_LINES, ROUTE_SEGMENTS } sweep_route[3] = {ROUTE_RULE, ROUTE_RULE, ROUTE_RULE};
   // hydrostatic background, FP64 (host + device copies)
   std::vector<double> hy_cells[3];     // dens, theta, pressure: [nz+2hs]
   std::vector<double> hy_edges[3];     // [nz+1]
