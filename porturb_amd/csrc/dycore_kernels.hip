@@ -416,7 +416,7 @@ static int sweep_x(pu_ctx *ctx, hipStream_t s, int stage, double dt, int nrelax)
   SweepParams P = sweep_params(ctx, 0);
   LaunchTimer lt(ctx, "weno_x");
   const dim3 blk(SX_BX, SX_BY, 1);
-  const dim3 grd((unsigned)((g.nx + SX_NC - 1) / SX_NC), (unsigned)((g.ny + SX_BY - 1) / SX_BY), (unsigned)g.nz);
+  const dim3 grd(x_blocks(g.nx, g.ny), 1, (unsigned)g.nz);
   const T *prim = (const T *)ctx->d_prim;
   T *tend = (T *)ctx->d_tend;
   FuseArgs<T> FA{};

@@ -700,8 +700,12 @@ void k_sweep_yline(const T *__restrict__ prim, const uint16_t *__restrict__ code
 }
 
 // ------------------------------------------------------------------------------------------------
-// x sweep (the last of a stage): a wave owns 64 consecutive cells of a row, 62 of them inner ones
-// plus one neighbour at each end whose reconstruction the end faces need.  Lane t computes the low
+// x sweep (the last of a stage): a wave owns 64 consecutive positions of a level's rows, 62 of them for
+// itself and one at each end whose reconstruction the end faces need.  A row is its cells and the
+// position before and after them, and the next row follows on in the same wave (x_position), so that rows
+// whose length is no multiple of 62 leave no lanes idle but the last wave's (us per launch, against waves
+// that end with their row: 64^3 order 5 31 -> 23.5, 150x70x51 order 7 62 -> 54, 512x512x128 order 9 4.22 ->
+// 4.06 ms; FP32 500x310x90 order 9 1358 -> 1240).  Lane t computes the low
 // face of its cell; upper values and fluxes pass between neighbouring lanes by wave shifts, so the
 // kernel has no LDS and no barrier and its waves run independently.
 // MODE 1 adds to the tendencies, MODE 2 takes each cell's finished tendency straight into the stage
@@ -709,6 +713,16 @@ void k_sweep_yline(const T *__restrict__ prim, const uint16_t *__restrict__ code
 // the stage-state reads and writes of the combination are coalesced.
 // ------------------------------------------------------------------------------------------------
 constexpr int SX_BX = 64, SX_BY = 4, SX_NC = SX_BX - 2;
+// waves of a level's positions, ny (nx + 2) without the first and the last
+inline unsigned x_blocks(int nx, int ny) { return (unsigned)(((ny * (nx + 2LL) - 2 + SX_NC - 1) / SX_NC + SX_BY - 1) / SX_BY); }
+// Row j and cell c (-1 .. n) of lane t of wave w of a level; j0: lane 0's row.
+__device__ __forceinline__ void x_position(int w, int t, int n, int &j0, int &j, int &c) {
+  const int f0 = w * SX_NC;
+  j = j0 = f0 / (n + 2);
+  c = f0 - j0 * (n + 2) + t;
+  while (c >= n + 2) { c -= n + 2; j++; }
+  c--;
+}
 
 // the value of the neighbouring lane below / above (wave shifts by one lane)
 template <int CTRL> __device__ __forceinline__ int wave_shift(int v) {
@@ -735,18 +749,23 @@ void k_sweep_x(const T *__restrict__ prim, const uint16_t *__restrict__ codes, T
   const int t = threadIdx.x, ty = __builtin_amdgcn_readfirstlane(threadIdx.y);
   unsigned bx, by, bz;
   swizzled_block(bx, by, bz);
-  const int c0 = (int)bx * SX_NC - 1, c = c0 + t, j = by * SX_BY + ty, k = bz, n = P.nx;
-  if (j >= P.ny) return;
+  const int k = bz, n = P.nx;
+  int j0, j, c;
+  x_position((int)bx * SX_BY + ty, t, n, j0, j, c);
+  if (j0 >= P.ny) return;
   const bool periodic = P.bc_along == PU_BC_PERIODIC;
-  const bool in_range = c <= n;
-  const bool do_recon = in_range && (periodic || (c >= 0 && c < n));
-  const bool has_face = in_range && t >= 1;
-  const bool has_tend = t >= 1 && t <= SX_NC && c < n;
+  const bool in_range = j < P.ny, inner = c >= 0 && c < n;
+  const bool do_recon = in_range && (periodic || inner);
+  const bool has_face = in_range && t >= 1 && c >= 0;
+  const bool has_tend = in_range && t >= 1 && t <= SX_NC && inner;
   const bool bface_lo = !periodic && c == 0, bface_hi = !periodic && c == n;
 
-  // first stencil point of the cell below lane 0's
-  const T *row = prim + ((long long)(k + hp) * P.nyh + (j + hp)) * P.nxh + (P.ox + c0 - hp);
-  const unsigned lane = (unsigned)(t * (int)sizeof(T));
+  // first stencil point of the cell below row j0's cell -1, and the lane's offset from there; the same of
+  // the cell arrays
+  const T *row = prim + ((long long)(k + hp) * P.nyh + (j0 + hp)) * P.nxh + (P.ox - 1 - hp);
+  const unsigned lane = (unsigned)(((j - j0) * (int)P.nxh + c + 1) * (int)sizeof(T));
+  const long long cell0 = ((long long)k * P.ny + j0) * P.nx - 1;
+  const unsigned clane = (unsigned)(((j - j0) * n + c + 1) * (int)sizeof(T));
   const long long crow = ((long long)k * P.ny + j) * P.nx;
   // a periodic neighbour cell past either end is the wrapped interior cell
   unsigned own = 0;
@@ -756,10 +775,9 @@ void k_sweep_x(const T *__restrict__ prim, const uint16_t *__restrict__ codes, T
 
   const T rd = (T)P.rd;
   const T hr = (T)P.hy_rc[hs + k], ht = (T)P.hy_tc[hs + k];
-  const long long cell0 = crow + c0;               // lane 0's cell
   StageIn S{0., 0., 0., 0., 0., 0.};
   if constexpr (MODE == 2) {
-    if (has_tend) S = stage_inputs(FA, cell0 + t, k);
+    if (has_tend) S = stage_inputs(FA, crow + c, k);
   }
   // the values a cell's finished tendency is combined with are loaded before the field's
   // reconstruction, so their latency hides behind it
@@ -767,10 +785,10 @@ void k_sweep_x(const T *__restrict__ prim, const uint16_t *__restrict__ codes, T
   auto prefetch = [&](int fidx) {
     Pre p{T(0), 0., 0.};
     if (has_tend) {
-      p.t = load_at<T, unsigned>(tend + ((long long)fidx * P.n3 + cell0), lane);
+      p.t = load_at<T, unsigned>(tend + ((long long)fidx * P.n3 + cell0), clane);
       if constexpr (MODE == 2) {
-        p.u = load_cons_at(FA.U, fidx, cell0, lane, P.n3);
-        if (FA.C.stage > 0) p.us = load_cons_at(FA.Us, fidx, cell0, lane, P.n3);
+        p.u = load_cons_at(FA.U, fidx, cell0, clane, P.n3);
+        if (FA.C.stage > 0) p.us = load_cons_at(FA.Us, fidx, cell0, clane, P.n3);
       }
     }
     return p;
@@ -780,10 +798,10 @@ void k_sweep_x(const T *__restrict__ prim, const uint16_t *__restrict__ codes, T
     const T v = -(from_lane_above(F) - F) * rd;
     if (!has_tend) return;
     if constexpr (MODE == 2)
-      store_at((FA.C.stage == 2 ? FA.U : FA.Us) + ((long long)fidx * P.n3 + cell0), lane,
+      store_at((FA.C.stage == 2 ? FA.U : FA.Us) + ((long long)fidx * P.n3 + cell0), clane,
                combine_value(FA.C, fidx, pf.t + v, pf.u, pf.us, S));
     else
-      store_at(tend + ((long long)fidx * P.n3 + cell0), lane, pf.t + v);
+      store_at(tend + ((long long)fidx * P.n3 + cell0), clane, pf.t + v);
   };
 
   // ---- phase A: density, u, pressure -> acoustic upwinding ----

@@ -442,8 +442,7 @@ void k_sweep_yline(const T *__restrict__ prim, const uint16_t *__restrict__ code
 }
 
 // Segment sweep: a 256-thread block covers line segments of BS-2 cells along the sweep plus one neighbour
-// cell at each end (the cell whose reconstruction the segment's end faces need).  x always (rows of
-// 64), y and z where the line kernels do not apply.  MODE: 0 writes the tendencies (z), 1 adds to them,
+// cell at each end (the cell whose reconstruction the segment's end faces need).  x always (its rows laid end to end, x_position), y and z where the line kernels do not apply.  MODE: 0 writes the tendencies (z), 1 adds to them,
 // 2 (x) takes each cell's finished tendency straight into the stage combination.
 template <int DIR> struct SegShape { static constexpr int BX = 8, BY = 32, BS = 32; };
 template <> struct SegShape<0> { static constexpr int BX = 64, BY = 4, BS = 64; };
@@ -470,7 +469,7 @@ void k_sweep(const T *__restrict__ prim, const uint16_t *__restrict__ codes,
   unsigned bx, by, bz;
   swizzled_block(bx, by, bz);
   int i, j, k, c, nal;
-  if (DIR == 0) { c = bx * NC - 1 + tx; i = c; j = by * BY + ty; k = bz; nal = P.nx; }
+  if (DIR == 0) { int j0; x_position((int)bx * BY + ty, tx, P.nx, j0, j, c); i = c; k = bz; nal = P.nx; }
   else if (DIR == 1) { i = bx * BX + tx; c = by * NC - 1 + ty; j = c; k = bz; nal = P.ny; }
   else { i = bx * BX + tx; j = by; c = bz * NC - 1 + ty; k = c; nal = P.nz; }
   const bool across_ok = DIR == 0 ? (j < P.ny) : (i < P.nx);
@@ -479,7 +478,7 @@ void k_sweep(const T *__restrict__ prim, const uint16_t *__restrict__ codes,
   const bool ghost = c < 0 || c >= nal;
   const bool do_recon = in_range && (!ghost || periodic);
   const bool has_face = in_range && t >= 1 && c >= 0;
-  const bool has_tend = in_range && t >= 1 && t <= NC && c < nal;
+  const bool has_tend = has_face && t <= NC && c < nal;
   const bool bface_lo = !periodic && c == 0;
   const bool bface_hi = !periodic && c == nal;
   const bool wallz = DIR == 2 && P.wall_z;

@@ -14,7 +14,8 @@ static void launch_ord(int dir, bool combine, hipStream_t s, const float *prim, 
   const dim3 bx(X::BX, X::BY), bl(L::BX, L::BY);
   const unsigned wx = (unsigned)((P.nx + L::BX - 1) / L::BX);
   if (dir == 0) {
-    const dim3 grd((unsigned)((P.nx + NX - 1) / NX), (unsigned)((P.ny + X::BY - 1) / X::BY), (unsigned)P.nz);
+    static_assert(X::BX == SX_BX && X::BY == SX_BY, "x_position");
+    const dim3 grd(x_blocks(P.nx, P.ny), 1, (unsigned)P.nz);
     if (combine) hipLaunchKernelGGL((f32::k_sweep<ORD, float, 0, 2>), grd, bx, 0, s, prim, codes, tend, P, FA);
     else hipLaunchKernelGGL((f32::k_sweep<ORD, float, 0, 1>), grd, bx, 0, s, prim, codes, tend, P, FA);
   } else if (dir == 1) {
