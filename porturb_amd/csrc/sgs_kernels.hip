@@ -71,6 +71,12 @@ __host__ __device__ constexpr int unit_of_k(int k) {
 
 // Hidden-layer activation: ReLU, and its derivative (0 at x = 0).
 __device__ __forceinline__ float relu(float x) { return fmaxf(x, 0.f); }
+// four values to bf16 (round to nearest even): two packed conversions
+__device__ __forceinline__ bfx4 bf16_bits4(fx4 v) {
+  typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(bfx4, __builtin_convertvector(v, bf16x4));
+}
+__device__ __forceinline__ bfx4 relu_bits4(fx4 v) { return bf16_bits4(fx4{relu(v[0]), relu(v[1]), relu(v[2]), relu(v[3])}); }
 __device__ __forceinline__ float relu_deriv(float x) { return x > 0.f ? 1.f : 0.f; }
 
 // sum over the 16 lanes that share l/16 (one column group of a D fragment)
@@ -520,59 +526,62 @@ template <class T> struct InferArgs {
   float4 *tau;          // [3][n3]: per face direction d, (tau_0d, tau_1d, tau_2d, q_d) of each cell
   unsigned char *flags;
 };
-// One group = 128 consecutive cells of an x row (i0..i0+127 at j, k); a block loops over groups.
-// The group's 3x3 neighbourhood rows of (u, v, w, theta), 130 x 3 x 3 points, are staged in LDS
+// One group = 128 consecutive cells of two x rows (i0..i0+127 at j, j+1 and k); a block loops over groups.
+// The group's neighbourhood rows of (u, v, w, theta), 130 x 4 x 3 points, are staged in LDS
 // with row-contiguous loads; each wave then takes 32 cells as two 16-cell tiles that share every
 // weight fragment it reads from LDS: inputs from LDS, the network on the matrix cores, the outputs
 // stored from the lanes that hold them in the last layer's D fragments, and (lanes 0-31, one cell
 // each) the fallback rule.
-constexpr int GX = 128, GBX = GX + 2, GBN = GBX * 3 * 3;
-
-// Waves per SIMD the inference kernel is built for (3: up to 168 VGPRs, no spills).
-#ifndef PU_SGS_INFER_WAVES
-#define PU_SGS_INFER_WAVES 3
-#endif
+// LDS reads and the inputs' arithmetic bound it, at few waves: two rows a block of eight waves share the
+// weights (two blocks, four waves per SIMD, in place of three of four waves) and a third of the staged
+// rows, and the weights' rows are padded so that the 16 lanes of a fragment read different banks (8-way
+// conflicts in layers 2 and 3 without).  512x256x128 in FP32: 1155 -> 1007 us; 500x310x90: 955 -> 820.
+constexpr int GX = 128, GY = 2, GBX = GX + 2, GBY = GY + 2, GBN = GBX * GBY * 3;
+constexpr int INFER_THREADS = 64 * GY * GX / 32;
+constexpr int LDW1 = NINP + 8, LDW2 = NH + 8;
 
 template <class T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PU_SGS_INFER_WAVES))) void k_sgs_infer(InferArgs<T> A) {
+__global__ __launch_bounds__(INFER_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_sgs_infer(InferArgs<T> A) {
   constexpr int K1 = 128;                       // layer-1 inputs: 4 K blocks of 32 (108 used)
-  __shared__ __align__(16) short sW1[NH * NINP];   // row stride 112: block 3 reads 16 columns
-  __shared__ __align__(16) short sW2[NH * NH];  // columns in unit_of_k order
-  __shared__ __align__(16) short sW3[NOUTP * NH];
+  __shared__ __align__(16) short sW1[NH * LDW1];   // block 3 reads 16 of the 112 columns
+  __shared__ __align__(16) short sW2[NH * LDW2];   // columns in unit_of_k order
+  __shared__ __align__(16) short sW3[NOUTP * LDW2];
   __shared__ __align__(16) float sB[NH + NH + NOUTP];
   __shared__ __align__(16) float sMS[2 * NOUTP];   // output mean, output scale (16 slots each)
-  __shared__ float sFm[K1];
+  __shared__ __align__(16) float sFm[K1];
   __shared__ T sQ[4 * GBN];                     // u, v, w, theta of the group's neighbourhood
   const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // the wave (uniform: row addresses are scalar)
-  for (int p = tid; p < NH * NINP / 4; p += 256)
-    reinterpret_cast<uint2 *>(sW1)[p] = reinterpret_cast<const uint2 *>(A.wbf + P_W1)[p];
-  for (int p = tid; p < NH * NH; p += 256) sW2[p] = A.wbf[P_W2 + (p / NH) * NH + unit_of_k(p % NH)];
-  for (int p = tid; p < NOUTP * NH; p += 256) sW3[p] = A.wbf[P_W3 + (p / NH) * NH + unit_of_k(p % NH)];
-  for (int p = tid; p < NH + NH + NOUTP; p += 256)
+  for (int p = tid; p < NH * NINP / 4; p += INFER_THREADS)
+    *reinterpret_cast<uint2 *>(sW1 + (p / (NINP / 4)) * LDW1 + 4 * (p % (NINP / 4))) = reinterpret_cast<const uint2 *>(A.wbf + P_W1)[p];
+  for (int p = tid; p < NH * NH; p += INFER_THREADS) sW2[(p / NH) * LDW2 + p % NH] = A.wbf[P_W2 + (p / NH) * NH + unit_of_k(p % NH)];
+  for (int p = tid; p < NOUTP * NH; p += INFER_THREADS) sW3[(p / NH) * LDW2 + p % NH] = A.wbf[P_W3 + (p / NH) * NH + unit_of_k(p % NH)];
+  for (int p = tid; p < NH + NH + NOUTP; p += INFER_THREADS)
     sB[p] = p < NH ? A.master[P_B1 + p] : (p < 2 * NH ? A.master[P_B2 + p - NH] : A.master[P_B3 + p - 2 * NH]);
-  for (int p = tid; p < K1; p += 256) sFm[p] = p < NIN ? A.fmul[p] : 0.f;
+  for (int p = tid; p < K1; p += INFER_THREADS) sFm[p] = p < NIN ? A.fmul[p] : 0.f;
   if (tid < NOUTP) {
     sMS[tid] = tid < NOUT ? A.out_mean[tid] : 0.f;
     sMS[NOUTP + tid] = tid < NOUT ? A.out_scale[tid] : 0.f;
   }
   // group bookkeeping in 32 bits (the host checks that the group count fits)
   const unsigned ngx = (unsigned)((A.nx + GX - 1) / GX);
-  const unsigned ngroups = ngx * (unsigned)A.ny * (unsigned)A.nz;
+  const unsigned ngy = (unsigned)((A.ny + GY - 1) / GY), ngroups = ngx * ngy * (unsigned)A.nz;
+  const int wx = w % (GX / 32), wy = w / (GX / 32);      // the wave's 32 cells: row j + wy, x from 32 wx
   for (unsigned grp = blockIdx.x; grp < ngroups; grp += gridDim.x) {
     const unsigned rest = grp / ngx;
-    const int i0 = (int)(grp - rest * ngx) * GX, j = (int)(rest % (unsigned)A.ny), k = (int)(rest / (unsigned)A.ny);
+    const int i0 = (int)(grp - rest * ngx) * GX, j0 = (int)(rest % ngy) * GY, k = (int)(rest / ngy), j = j0 + wy;
     const int lxmax = (int)(A.nxh - i0);        // box x positions inside the array
-    // Staging: the box is 36 rows (quantity q, z offset, y offset) of 130 points; wave w loads rows
-    // w, w+4, ... with one lane per x point (points lane, 64 + lane; lanes 0, 1 also 128, 129), so
-    // each row's address is wave-uniform.  All loads are issued before any LDS write.
-    constexpr int RPW = 36 / 4;
+    // Staging: the box is 48 rows (quantity q, z offset, y offset) of 130 points; wave w loads rows
+    // w, w+8, ... with one lane per x point (points lane, 64 + lane; lanes 0, 1 also 128, 129), so
+    // each row's address is wave-uniform.  All loads are issued before any LDS write.  A row past the
+    // array (the last group of an odd ny) belongs to no cell inside and repeats the last one.
+    constexpr int NW = INFER_THREADS / 64, RPW = 4 * 3 * GBY / NW;
     T buf[RPW], buf2[RPW], buf3[RPW];
+    const int jr = min(j0 + w % GBY, (int)A.nyh - 1);        // the wave's rows share their y offset
 #pragma unroll
     for (int rr = 0; rr < RPW; rr++) {
-      const int r = w + 4 * rr;
-      const int q = r / 9, lz = (r / 3) % 3, ly = r % 3;
-      const T *row = A.F + (long long)(1 + q) * A.nh + ((long long)(k + lz) * A.nyh + (j + ly)) * A.nxh + i0;
+      const int ql = (w + NW * rr) / GBY, q = ql / 3, lz = ql % 3;
+      const T *row = A.F + (long long)(1 + q) * A.nh + ((long long)(k + lz) * A.nyh + jr) * A.nxh + i0;
       buf[rr] = lane < lxmax ? row[lane] : T(0);
       buf2[rr] = 64 + lane < lxmax ? row[64 + lane] : T(0);
       buf3[rr] = (lane < 2 && 128 + lane < lxmax) ? row[128 + lane] : T(0);
@@ -580,7 +589,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PU_SGS_INFE
     __syncthreads();                            // the previous group is done with sQ
 #pragma unroll
     for (int rr = 0; rr < RPW; rr++) {
-      const int r = w + 4 * rr;
+      const int r = w + NW * rr;
       sQ[r * GBX + lane] = buf[rr];
       sQ[r * GBX + 64 + lane] = buf2[rr];
       if (lane < 2) sQ[r * GBX + 128 + lane] = buf3[rr];
@@ -592,7 +601,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PU_SGS_INFE
     float mxt[2] = {0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < 2; t++) {
-      const int c = (1 * 3 + 1) * GBX + 32 * w + 16 * t + r16 + 1;   // the cell's index in the staged box
+      const int c = (GBY + 1 + wy) * GBX + 32 * wx + 16 * t + r16 + 1;   // the cell's index in the staged box
 #pragma unroll
       for (int kb = 0; kb < 4; kb++) {
         bfx8 v = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -601,13 +610,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PU_SGS_INFE
           const int n = 8 * kb + 2 * g + h;
           if (n < 27) {
             const int dz = n / 9 - 1, dy = (n / 3) % 3 - 1, dx = n % 3 - 1;
-            const int nb = c + (dz * 3 + dy) * GBX + dx;
+            const int nb = c + (dz * GBY + dy) * GBX + dx;
+            fx4 x;
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-              const float x = (float)(sQ[q * GBN + nb] - sQ[q * GBN + c]) * sFm[4 * n + q];
-              mxt[t] = fmaxf(mxt[t], fabsf(x));
-              v[4 * h + q] = bf16_bits(x);
+              x[q] = (float)(sQ[q * GBN + nb] - sQ[q * GBN + c]) * sFm[4 * n + q];
+              mxt[t] = fmaxf(mxt[t], fabsf(x[q]));
             }
+            const bfx4 b = bf16_bits4(x);
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[4 * h + q] = b[q];
           }
         }
         xb[t][kb] = v;
@@ -628,15 +640,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PU_SGS_INFE
 #pragma unroll
       for (int kb = 0; kb < 4; kb++) {
         // inputs 112..127 do not exist (their B values are 0): lanes 32..63 of block 3 use a zero A
-        const bfx8 wa = (kb == 3 && g >= 2) ? bfx8{0, 0, 0, 0, 0, 0, 0, 0} : ld8(sW1 + (16 * mt + r16) * NINP + 32 * kb + 8 * g);
+        const bfx8 wa = (kb == 3 && g >= 2) ? bfx8{0, 0, 0, 0, 0, 0, 0, 0} : ld8(sW1 + (16 * mt + r16) * LDW1 + 32 * kb + 8 * g);
         acc0 = mfma32(wa, xb[0][kb], acc0);
         acc1 = mfma32(wa, xb[1][kb], acc1);
       }
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        a1[0][mt][r] = bf16_bits(relu(acc0[r]));
-        a1[1][mt][r] = bf16_bits(relu(acc1[r]));
-      }
+      a1[0][mt] = relu_bits4(acc0);
+      a1[1][mt] = relu_bits4(acc1);
     }
     // layer 2: the B fragment of K block kb2 is (a1[2 kb2], a1[2 kb2 + 1]) in unit_of_k order
 #pragma unroll
@@ -645,21 +654,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PU_SGS_INFE
       fx4 acc0 = bias, acc1 = bias;
 #pragma unroll
       for (int kb = 0; kb < 2; kb++) {
-        const bfx8 wa = ld8(sW2 + (16 * mt + r16) * NH + 32 * kb + 8 * g);
+        const bfx8 wa = ld8(sW2 + (16 * mt + r16) * LDW2 + 32 * kb + 8 * g);
         acc0 = mfma32(wa, cat8(a1[0][2 * kb], a1[0][2 * kb + 1]), acc0);
         acc1 = mfma32(wa, cat8(a1[1][2 * kb], a1[1][2 * kb + 1]), acc1);
       }
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        a2[0][mt][r] = bf16_bits(relu(acc0[r]));
-        a2[1][mt][r] = bf16_bits(relu(acc1[r]));
-      }
+      a2[0][mt] = relu_bits4(acc0);
+      a2[1][mt] = relu_bits4(acc1);
     }
     const fx4 b3 = *reinterpret_cast<const fx4 *>(sB + 2 * NH + 4 * g);
     fx4 y0 = b3, y1 = b3;
 #pragma unroll
     for (int kb = 0; kb < 2; kb++) {
-      const bfx8 wa = ld8(sW3 + r16 * NH + 32 * kb + 8 * g);
+      const bfx8 wa = ld8(sW3 + r16 * LDW2 + 32 * kb + 8 * g);
       y0 = mfma32(wa, cat8(a2[0][2 * kb], a2[0][2 * kb + 1]), y0);
       y1 = mfma32(wa, cat8(a2[1][2 * kb], a2[1][2 * kb + 1]), y1);
     }
@@ -688,19 +694,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PU_SGS_INFE
       t[8] = g == 0 ? c0 : c1;
     }
     const float mxl = g == 0 ? mxt[0] : mxt[1];
-    const int xl = 32 * w + lane;                // this lane's cell (lanes 0..31)
+    const int xl = 32 * wx + lane;               // this lane's cell (lanes 0..31)
     const int i = i0 + xl;
-    if (lane < 32 && i < A.nx) {
+    if (lane < 32 && i < A.nx && j < A.ny) {
       const long long id = idrow + i;
       // outputs t = (tau11, tau12, tau13, tau22, tau23, tau33, q1, q2, q3)
       A.tau[id] = make_float4(t[0], t[1], t[2], t[6]);
       A.tau[A.n3 + id] = make_float4(t[1], t[3], t[4], t[7]);
       A.tau[2 * A.n3 + id] = make_float4(t[2], t[4], t[5], t[8]);
-      const int c = (1 * 3 + 1) * GBX + xl + 1;
+      const int c = (GBY + 1 + wy) * GBX + xl + 1;
       unsigned char fl = 0;
       if (A.valid[id] && mxl <= A.xmax) {
         const T *U = sQ, *V = sQ + GBN, *W = sQ + 2 * GBN, *TH = sQ + 3 * GBN;
-        const int sy = GBX, sz = 3 * GBX;
+        const int sy = GBX, sz = GBY * GBX;
         const double ux = (U[c + 1] - U[c - 1]) * A.r2dx, uy = (U[c + sy] - U[c - sy]) * A.r2dy, uz = (U[c + sz] - U[c - sz]) * A.r2dz;
         const double vx = (V[c + 1] - V[c - 1]) * A.r2dx, vy = (V[c + sy] - V[c - sy]) * A.r2dy, vz = (V[c + sz] - V[c - sz]) * A.r2dz;
         const double wx = (W[c + 1] - W[c - 1]) * A.r2dx, wy = (W[c + sy] - W[c - sy]) * A.r2dy, wz = (W[c + sz] - W[c - sz]) * A.r2dz;
@@ -830,10 +836,10 @@ static int sgs_infer_t(pu_ctx *ctx, double dt) {
   const double vmx = 0.25 * dx * dx / dt, vmy = 0.25 * dy * dy / dt, vmz = 0.25 * dz * dz / dt;
   A.nu_max = 0.5 * std::fmin(vmx, std::fmin(vmy, vmz));
   A.tau = reinterpret_cast<float4 *>(ctx->d_sgs_tau); A.flags = ctx->d_sgs_flags;
-  const long long ngroups = (long long)((c.nx + GX - 1) / GX) * c.ny * c.nz;
+  const long long ngroups = (long long)((c.nx + GX - 1) / GX) * ((c.ny + GY - 1) / GY) * c.nz;
   if (ngroups >= (1LL << 32)) return fail(PU_ERR_UNSUPPORTED, "learned closure: grid too large for the inference kernel");
-  const unsigned grid = (unsigned)std::min<long long>(ngroups, 256LL * 16);
-  hipLaunchKernelGGL(k_sgs_infer<T>, dim3(grid), dim3(256), 0, ctx->stream, A);
+  const unsigned grid = (unsigned)std::min<long long>(ngroups, 256LL * 8);
+  hipLaunchKernelGGL(k_sgs_infer<T>, dim3(grid), dim3(INFER_THREADS), 0, ctx->stream, A);
   PU_HIP_CHECK(hipGetLastError());
   return PU_OK;
 }

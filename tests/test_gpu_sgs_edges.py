@@ -1,0 +1,35 @@
+"""Inference kernel at the edges of its groups of two rows of 128 cells (a last row of its own, one cell
+past a group, a last tile of one cell), both precisions, against the oracle.
+
+Bounds: the median of an output 1e-4 and its largest error 2e-2 of the output's largest; both sides round
+inputs and activations to bf16 from sums in another order (2^-8 of one of 64 terms)."""
+import numpy as np
+import pytest
+
+import porturb_amd as pa
+from oracle import oracle_py as o
+from tests.helpers import random_state, small_config, WV, TKE, P1, P2
+from tests.test_gpu_sgs import model_for, rand_params, run_learned
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("precision", [pa.PU_FP64, pa.PU_FP32], ids=["fp64", "fp32"])
+@pytest.mark.parametrize("size", [(129, 7, 6), (128, 9, 5), (17, 5, 8), (255, 8, 5)], ids=str)
+def test_inference_at_group_edges(size, precision):
+    nx, ny, nz = size
+    cfg = small_config(nx=nx, ny=ny, nz=nz, ord=5, tracers=[WV, TKE, P1, P2], dx=2., precision=precision)
+    st, imm = random_state(cfg, seed=27, buildings=1, amp_u=1.0)
+    print("case", size, precision, flush=True)
+    P = rand_params(28, scale=0.1)
+    om = np.array([0.02, 0, -0.01, 0.02, 0, 0.02, 0, 0, -1e-3], np.float32)
+    os_ = np.array([0.01, 0.005, 0.005, 0.01, 0.005, 0.01, 1e-3, 1e-3, 1e-3], np.float32)
+    gm, om_ = model_for(P, om, os_)
+    _, tau, fl = run_learned(cfg, st, imm, gm, 0.02)
+    rtau, rfl = o.les_apply_learned(cfg, st.copy(), imm, 0.02, om_)
+    assert (fl == rfl).mean() >= 0.99
+    for f in range(9):
+        s = max(np.abs(rtau[f]).max(), 1e-30)
+        err = np.abs(tau[f] - rtau[f])
+        assert np.median(err) <= 1e-4 * s and err.max() <= 2e-2 * s, f
+    gm.destroy()
