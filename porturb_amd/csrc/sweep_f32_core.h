@@ -442,7 +442,9 @@ void k_sweep_yline(const T *__restrict__ prim, const uint16_t *__restrict__ code
 }
 
 // Segment sweep: a 256-thread block covers line segments of BS-2 cells along the sweep plus one neighbour
-// cell at each end (the cell whose reconstruction the segment's end faces need).  x always (its rows laid end to end, x_position), y and z where the line kernels do not apply.  MODE: 0 writes the tendencies (z), 1 adds to them,
+// cell at each end (the cell whose reconstruction the segment's end faces need).  x always (its rows laid
+// end to end, x_position; neighbours by wave shifts: 2 % less than through LDS with two barriers a field),
+// y and z where the line kernels do not apply.  MODE: 0 writes the tendencies (z), 1 adds to them,
 // 2 (x) takes each cell's finished tendency straight into the stage combination.
 template <int DIR> struct SegShape { static constexpr int BX = 8, BY = 32, BS = 32; };
 template <> struct SegShape<0> { static constexpr int BX = 64, BY = 4, BS = 64; };
@@ -452,6 +454,12 @@ template <> struct SegShape<0> { static constexpr int BX = 64, BY = 4, BS = 64; 
 #ifndef PU_X_F32_WAVES
 #define PU_X_F32_WAVES 6
 #endif
+// a - b, never fused with the product that made one of them
+template <class T> __device__ __forceinline__ T plain_difference(T a, T b) {
+#pragma clang fp contract(off)
+  return a - b;
+}
+
 template <int ORD, class T, int DIR, int MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIR == 0 ? PU_X_F32_WAVES : 1)))
 void k_sweep(const T *__restrict__ prim, const uint16_t *__restrict__ codes,
@@ -461,7 +469,9 @@ void k_sweep(const T *__restrict__ prim, const uint16_t *__restrict__ codes,
   constexpr int BX = SegShape<DIR>::BX, BY = SegShape<DIR>::BY, BS = SegShape<DIR>::BS;
   constexpr int NC = BS - 2;
   constexpr int NT = BX * BY;
-  __shared__ T bufA0[NT], bufA1[NT], bufA2[NT], bufB0[NT], bufB1[NT];
+  // x: a wave is a row and neighbours pass values by wave shifts; y and z: through LDS
+  constexpr int NS = DIR == 0 ? 1 : NT;
+  __shared__ T bufA0[NS], bufA1[NS], bufA2[NS], bufB0[NS], bufB1[NS];
 
   const int tx = threadIdx.x, ty = threadIdx.y, lin = ty * BX + tx;
   const int t = DIR == 0 ? tx : ty;
@@ -538,12 +548,17 @@ void k_sweep(const T *__restrict__ prim, const uint16_t *__restrict__ codes,
     recon(ln, false, qLu, qRu);
     recon(idP, true, qLp, qRp);
   }
-  bufA0[lin] = qRr; bufA1[lin] = qRu; bufA2[lin] = qRp;
-  __syncthreads();
+  T rL = 0, uL = 0, pL = 0;
+  if constexpr (DIR == 0) {
+    rL = from_lane_below(qRr); uL = from_lane_below(qRu); pL = from_lane_below(qRp);
+  } else {
+    bufA0[lin] = qRr; bufA1[lin] = qRu; bufA2[lin] = qRp;
+    __syncthreads();
+    if (has_face) { rL = bufA0[lin - nbs]; uL = bufA1[lin - nbs]; pL = bufA2[lin - nbs]; }
+  }
   Upw<T> up{T(0), T(0), true};
   T Fr = 0, Fu = 0;
   if (has_face) {
-    T rL = bufA0[lin - nbs], uL = bufA1[lin - nbs], pL = bufA2[lin - nbs];
     T rR = qLr, uR = qLu, pR = qLp;
     if (bface_lo) { rL = rR; uL = uR; pL = pR; }
     if (bface_hi) { rR = rL; uR = uL; pR = pL; }
@@ -552,11 +567,16 @@ void k_sweep(const T *__restrict__ prim, const uint16_t *__restrict__ codes,
     Fr = up.ru;
     Fu = up.ru * (up.left ? uL : uR) + up.p;
   }
-  bufB0[lin] = Fr; bufB1[lin] = Fu;
-  __syncthreads();
+  // x: the flux through the cell's high face less the one through its low face
+  auto difference = [&](T F) { return plain_difference(from_lane_above(F), F); };
+  if constexpr (DIR != 0) {
+    bufB0[lin] = Fr; bufB1[lin] = Fu;
+    __syncthreads();
+  }
+  const T dr = DIR == 0 ? difference(Fr) : T(0), du = DIR == 0 ? difference(Fu) : T(0);
   if (has_tend) {
-    accumulate(idR, -(bufB0[lin + nbs] - bufB0[lin]) * rd);
-    accumulate(ln, -(bufB1[lin + nbs] - bufB1[lin]) * rd);
+    accumulate(idR, -(DIR == 0 ? dr : bufB0[lin + nbs] - bufB0[lin]) * rd);
+    accumulate(ln, -(DIR == 0 ? du : bufB1[lin + nbs] - bufB1[lin]) * rd);
   }
 
   // ---- phase B: the advected fields, one at a time ----
@@ -572,20 +592,31 @@ void k_sweep(const T *__restrict__ prim, const uint16_t *__restrict__ codes,
     else { l = NUM_STATE + 1 + (b - 3); fidx = NUM_STATE + (b - 3); }
     T qL = 0, qR = 0;
     if (do_recon) recon(l, modify, qL, qR);
-    bufA0[lin] = qR;
-    __syncthreads();
+    T vL = 0;
+    if constexpr (DIR == 0) {
+      vL = from_lane_below(qR);
+    } else {
+      bufA0[lin] = qR;
+      __syncthreads();
+      if (has_face) vL = bufA0[lin - nbs];
+    }
     T F = 0;
     if (has_face) {
-      T vL = bufA0[lin - nbs], vR = qL;
+      T vR = qL;
       if (bface_lo) vL = vR;
       if (bface_hi) vR = vL;
       if (wallz && (bface_lo || bface_hi) && l == idT) { vL = 0; vR = 0; }
       if (l == idT) { vL += ht; vR += ht; }
       F = up.ru * (up.left ? vL : vR);
     }
-    bufB0[lin] = F;
-    __syncthreads();
-    if (has_tend) accumulate(fidx, -(bufB0[lin + nbs] - bufB0[lin]) * rd);
+    if constexpr (DIR == 0) {
+      const T dF = difference(F);
+      if (has_tend) accumulate(fidx, -dF * rd);
+    } else {
+      bufB0[lin] = F;
+      __syncthreads();
+      if (has_tend) accumulate(fidx, -(bufB0[lin + nbs] - bufB0[lin]) * rd);
+    }
   }
 }
 
