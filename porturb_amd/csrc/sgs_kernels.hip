@@ -407,14 +407,19 @@ struct FilterArgs {
   float *targets;
 };
 
-__global__ __launch_bounds__(256) void k_sgs_filter(FilterArgs A) {
-  const long long id = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (id >= A.n3c) return;
+// LANES threads per coarse cell: two for even ratios from 4 on, each with one half of the fine cells in x,
+// so that the chain of r^3 powers of a thread is half as long (us, one thread and two: 384x256x96 by 4
+// 166, 139; 384x256x128 by 2, eight powers, 187, 192).
+template <int LANES> __global__ __launch_bounds__(256) void k_sgs_filter(FilterArgs A) {
+  const long long t = (long long)blockIdx.x * 256 + threadIdx.x, id = t / LANES;
+  const int half = (int)(t % LANES);
+  if (id >= A.n3c) return;                                    // the lanes of a cell leave together
   const int I = (int)(id % A.nxc), J = (int)((id / A.nxc) % A.nyc), K = (int)(id / ((long long)A.nxc * A.nyc));
   double m[5] = {0, 0, 0, 0, 0}, uu[6] = {0, 0, 0, 0, 0, 0}, ut[3] = {0, 0, 0}, im = 0;
+  const int e0 = half * (A.r / LANES), e1 = e0 + A.r / LANES;
   for (int a = 0; a < A.r; a++)
     for (int b = 0; b < A.r; b++)
-      for (int e = 0; e < A.r; e++) {
+      for (int e = e0; e < e1; e++) {
         const long long f = ((long long)(K * A.r + a) * A.ny + (J * A.r + b)) * A.nx + (I * A.r + e);
         const double rho = A.rho[f], u = A.u[f], v = A.v[f], w = A.w[f];
         const double th = pow_pos(rho * A.R_d * A.T[f] / A.C0, A.inv_gamma) / rho;
@@ -424,18 +429,24 @@ __global__ __launch_bounds__(256) void k_sgs_filter(FilterArgs A) {
         im = fmax(im, A.imm[f]);
       }
   const double inv = 1. / ((double)A.r * A.r * A.r);
-  for (int f = 0; f < 5; f++) m[f] *= inv;
-  for (int f = 0; f < 6; f++) uu[f] *= inv;
-  for (int f = 0; f < 3; f++) ut[f] *= inv;
+  auto total = [&](double x) { return LANES == 2 ? x + __shfl_xor(x, 1) : x; };
+  for (int f = 0; f < 5; f++) m[f] = total(m[f]) * inv;
+  for (int f = 0; f < 6; f++) uu[f] = total(uu[f]) * inv;
+  for (int f = 0; f < 3; f++) ut[f] = total(ut[f]) * inv;
+  if (LANES == 2) im = fmax(im, __shfl_xor(im, 1));
   const double tau[6] = {uu[0] - m[1] * m[1], uu[1] - m[1] * m[2], uu[2] - m[1] * m[3],
                          uu[3] - m[2] * m[2], uu[4] - m[2] * m[3], uu[5] - m[3] * m[3]};
   const double q[3] = {ut[0] - m[1] * m[4], ut[1] - m[2] * m[4], ut[2] - m[3] * m[4]};
   const long long h = ((long long)(K + 1) * A.nyh + (J + 1)) * A.nxh + (I + 1);
-  for (int f = 0; f < 5; f++) A.les[f * A.nh + h] = m[f];
-  A.les[5 * A.nh + h] = 0.5 * (tau[0] + tau[3] + tau[5]);
-  A.immc[h] = im;
-  for (int f = 0; f < 6; f++) A.targets[f * A.n3c + id] = (float)tau[f];
-  for (int f = 0; f < 3; f++) A.targets[(6 + f) * A.n3c + id] = (float)q[f];
+  if (half == 0) {
+    for (int f = 0; f < 5; f++) A.les[f * A.nh + h] = m[f];
+    A.les[5 * A.nh + h] = 0.5 * (tau[0] + tau[3] + tau[5]);
+    A.immc[h] = im;
+  }
+  if (half == LANES - 1) {
+    for (int f = 0; f < 6; f++) A.targets[f * A.n3c + id] = (float)tau[f];
+    for (int f = 0; f < 3; f++) A.targets[(6 + f) * A.n3c + id] = (float)q[f];
+  }
 }
 
 // halo of the filtered box: x/y periodic (corners wrap both), z copies with w = 0, immersed 1
@@ -1038,7 +1049,10 @@ int pu_sgs_filter(pu_ctx *ctx, const pu_coupler_state *cs, int r, double *les, d
   A.nxh = A.nxc + 2; A.nyh = A.nyc + 2; A.nh = A.nxh * A.nyh * (A.nzc + 2);
   A.R_d = c.R_d; A.C0 = c.C0; A.inv_gamma = 1. / c.gamma_d;
   A.les = les; A.immc = imm; A.targets = targets;
-  hipLaunchKernelGGL(k_sgs_filter, dim3((unsigned)((A.n3c + 255) / 256)), dim3(256), 0, ctx->stream, A);
+  if (A.r % 2 == 0 && A.r >= 4)
+    hipLaunchKernelGGL(k_sgs_filter<2>, dim3((unsigned)((2 * A.n3c + 255) / 256)), dim3(256), 0, ctx->stream, A);
+  else
+    hipLaunchKernelGGL(k_sgs_filter<1>, dim3((unsigned)((A.n3c + 255) / 256)), dim3(256), 0, ctx->stream, A);
   PU_HIP_CHECK(hipGetLastError());
   hipLaunchKernelGGL(k_sgs_filter_halo, dim3((unsigned)((A.nh + 255) / 256)), dim3(256), 0, ctx->stream, A);
   PU_HIP_CHECK(hipGetLastError());

@@ -9,7 +9,7 @@ import pytest
 import porturb_amd as pa
 from oracle import oracle_py as o
 from tests.helpers import random_state, small_config, WV, TKE, P1, P2
-from tests.test_gpu_sgs import model_for, rand_params, run_learned
+from tests.test_gpu_sgs import fine_state, model_for, rand_params, run_learned
 
 pytestmark = pytest.mark.gpu
 
@@ -33,3 +33,23 @@ def test_inference_at_group_edges(size, precision):
         err = np.abs(tau[f] - rtau[f])
         assert np.median(err) <= 1e-4 * s and err.max() <= 2e-2 * s, f
     gm.destroy()
+
+
+@pytest.mark.parametrize("ratio,n", [(2, (17, 9, 5)), (3, (11, 7, 4)), (4, (13, 11, 3)), (6, (5, 3, 4))], ids=str)
+def test_filter_ratios(ratio, n):
+    """Box filter with one and with two threads a coarse cell, cells that do not fill a block.  Bounds as at
+    ratio 2: 1e-12 of a field (sums of up to 216 terms in another order), 1e-6 of a float target."""
+    nx, ny, nz = n
+    cfg, st, imm = fine_state(ratio * nx, ratio * ny, ratio * nz)
+    print("case", ratio, n, flush=True)
+    cs = pa.CouplerState(cfg)
+    cs.upload((st, imm))
+    d = pa.Dycore(cfg)
+    les, immc, tg = pa.sgs_filter(d.ctx, cs.c, cfg, ratio)
+    r_les, r_imm, r_tg = o.sgs_filter(cfg, st, imm, ratio)
+    assert np.array_equal(immc.download(np.float64, (nz + 2, ny + 2, nx + 2)), r_imm)
+    g_les, g_tg = les.download(np.float64, (6, nz + 2, ny + 2, nx + 2)), tg.download(np.float32, (9, nz, ny, nx))
+    for f in range(6):
+        assert np.abs(g_les[f] - r_les[f]).max() <= 1e-12 * max(np.abs(r_les[f]).max(), 1e-30), f
+    for f in range(9):
+        assert np.abs(g_tg[f] - r_tg[f]).max() <= 1e-6 * max(np.abs(r_tg[f]).max(), 1e-30), f
