@@ -35,7 +35,8 @@ __global__ __launch_bounds__(256) void k_sfc_halo(const double *__restrict__ f3,
 struct SfcParams {
   int nx, ny, nz;
   double dx, dy, dz, dt;
-  const double *prop, *rough, *temp;    // halo'd boxes
+  const unsigned char *code;            // immersed proportion of the halo'd box: 0 none, 1 partial, 2 full
+  const double *rough, *temp;           // halo'd boxes
 };
 
 // grid: (blocks over one level's nx*ny cells, nz levels): no 64-bit division for the indices
@@ -48,17 +49,18 @@ __global__ __launch_bounds__(256) void k_surface_fluxes(double *uu, double *vv, 
   const long long nxh = P.nx + 2, nyh = P.ny + 2;
   const long long c = ((long long)(k + 1) * nyh + (j + 1)) * nxh + (i + 1);
   // a cell without an immersed face neighbour has zero tendencies: it is left as it is (u + dt*0
-  // is u), so most of the domain reads only the immersed proportions and writes nothing
+  // is u), so most of the domain reads only the immersed codes and writes nothing
   const long long sz = nxh * nyh;
-  if (!(P.prop[c - 1] > 0 || P.prop[c + 1] > 0 || P.prop[c - nxh] > 0 || P.prop[c + nxh] > 0 ||
-        P.prop[c - sz] > 0 || P.prop[c + sz] > 0))
-    return;
+  // Their codes (bytes, 0: none) are loaded together, then tested.  512x512x128: 238 us with the proportions
+  // as doubles one after the other, as || does it, 181 with the six in flight, 129 with the bytes.
+  const unsigned char ib[6] = {P.code[c - 1], P.code[c + 1], P.code[c - nxh], P.code[c + nxh], P.code[c - sz], P.code[c + sz]};
+  if ((ib[0] | ib[1] | ib[2] | ib[3] | ib[4] | ib[5]) == 0) return;
   const double u = uu[id], v = vv[id], w = ww[id], T = tt[id];
   const double vk = 0.40;
   double tu = 0, tv = 0, tw = 0, tT = 0;
   // one immersed neighbour across a face normal to `dir` (0 x, 1 y, 2 z)
-  auto face = [&](long long nb, int dir) {
-    if (!(P.prop[nb] > 0)) return;
+  auto face = [&](int f, long long nb, int dir) {
+    if (!ib[f]) return;
     const double delta = dir == 0 ? P.dx : (dir == 1 ? P.dy : P.dz);
     const double z0 = P.rough[nb];
     const double lg = log((delta / 2 + z0) / z0);
@@ -81,12 +83,12 @@ __global__ __launch_bounds__(256) void k_surface_fluxes(double *uu, double *vv, 
       if (T0 != 0) tT += -cd * (T - T0) * mag / delta;
     }
   };
-  face(c - 1, 0);
-  face(c + 1, 0);
-  face(c - nxh, 1);
-  face(c + nxh, 1);
-  face(c - nxh * nyh, 2);
-  face(c + nxh * nyh, 2);
+  face(0, c - 1, 0);
+  face(1, c + 1, 0);
+  face(2, c - nxh, 1);
+  face(3, c + nxh, 1);
+  face(4, c - nxh * nyh, 2);
+  face(5, c + nxh * nyh, 2);
   uu[id] = u + P.dt * tu;
   vv[id] = v + P.dt * tv;
   ww[id] = w + P.dt * tw;
@@ -130,7 +132,7 @@ int pu_surface_fluxes_apply(pu_ctx *ctx, pu_coupler_state *cs, double dt_phys) {
   SfcParams P;
   P.nx = c.nx; P.ny = c.ny; P.nz = c.nz;
   P.dx = c.xlen / c.nx; P.dy = c.ylen / c.ny; P.dz = c.zlen / c.nz; P.dt = dt_phys;
-  P.prop = ctx->d_imm_les_val; P.rough = ctx->d_sfc_rough; P.temp = ctx->d_sfc_temp;
+  P.code = ctx->d_imm_les; P.rough = ctx->d_sfc_rough; P.temp = ctx->d_sfc_temp;
   {
     LaunchTimer lt(ctx, "surface");
     hipLaunchKernelGGL(k_surface_fluxes, dim3((unsigned)((c.nx * c.ny + 255) / 256), (unsigned)c.nz), dim3(256), 0,
