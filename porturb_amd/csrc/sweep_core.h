@@ -709,7 +709,7 @@ void k_sweep_yline(const T *__restrict__ prim, const uint16_t *__restrict__ code
 // face of its cell; upper values and fluxes pass between neighbouring lanes by wave shifts, so the
 // kernel has no LDS and no barrier and its waves run independently.
 // MODE 1 adds to the tendencies, MODE 2 takes each cell's finished tendency straight into the stage
-// combination (combine_field_v).  The stage runs z, y, x: this sweep's rows are 64 cells wide, so
+// combination (combine_value).  The stage runs z, y, x: this sweep's waves take 64 cells of a row, so
 // the stage-state reads and writes of the combination are coalesced.
 // ------------------------------------------------------------------------------------------------
 constexpr int SX_BX = 64, SX_BY = 4, SX_NC = SX_BX - 2;

@@ -1,5 +1,5 @@
 // sweep_f32_core.h -- the FP32 sweep kernels: the segment sweep k_sweep, the whole-column z sweep
-// k_sweep_zwall and the whole-line y sweep k_sweep_pline.  Every field is reconstructed on both sides of
+// k_sweep_zwall and the whole-line y sweep k_sweep_yline.  Every field is reconstructed on both sides of
 // a cell from its stencil in memory order.  The upwind-side evaluation of the FP64 sweeps
 // (sweep_core.h), which reads half of the stencils in reverse, is not used in FP32: the limiter's map
 // turns one rounding of a velocity (5e-7 at 8 m/s) into up to 4e-5 where a weight sits on its steep part,
@@ -449,8 +449,7 @@ void k_sweep_yline(const T *__restrict__ prim, const uint16_t *__restrict__ code
 template <int DIR> struct SegShape { static constexpr int BX = 8, BY = 32, BS = 32; };
 template <> struct SegShape<0> { static constexpr int BX = 64, BY = 4, BS = 64; };
 
-// x: at most 80 VGPRs (6 waves per SIMD; 3.13 ms per launch at 512x512x128, 3.14 at 72 VGPRs, 3.25 at 64,
-// where it spills)
+// x: at most 80 VGPRs (6 waves per SIMD): 2.93 ms per launch at 512x512x128; 72 VGPRs run the same
 #ifndef PU_X_F32_WAVES
 #define PU_X_F32_WAVES 6
 #endif
