@@ -298,7 +298,7 @@ __global__ __launch_bounds__(LES_THREADS) void k_les_update(const T *__restrict_
   long long goff[PER];
 #pragma unroll
   for (int e = 0; e < PER; e++) {
-    const BoxPoint b(threadIdx.x + LES_THREADS * e);
+    const BoxPoint b(min((int)threadIdx.x + LES_THREADS * e, NB - 1));
     const int ih = min(i0 + b.i, (int)P.nxh - 1), jh = min(j0 + b.j, (int)P.nyh - 1), kh = min(k0 + b.k, (int)P.nzh - 1);
     goff[e] = ((long long)kh * (int)P.nyh + jh) * (int)P.nxh + ih;
   }
