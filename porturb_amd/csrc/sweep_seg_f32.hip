@@ -10,7 +10,7 @@ static void launch_ord(int dir, bool combine, hipStream_t s, const float *prim, 
                        const SweepParams &P, const FuseArgs<float> &FA) {
   using X = f32::SegShape<0>;
   using L = f32::SegShape<1>;
-  constexpr int NX = X::BS - 2, NL = L::BS - 2;
+  constexpr int NL = L::BS - 2;
   const dim3 bx(X::BX, X::BY), bl(L::BX, L::BY);
   const unsigned wx = (unsigned)((P.nx + L::BX - 1) / L::BX);
   if (dir == 0) {
