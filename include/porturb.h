@@ -416,6 +416,12 @@ int  pu_les_closure_sgs(pu_ctx *ctx, const pu_coupler_state *cs, double dt_phys,
 int  pu_measure_fma_rate(int precision, double *tflops);
 int  pu_measure_copy_rate(size_t bytes, double *gbps);
 
+/* The square root (PU_FN_ROOT) or power x^a (PU_FN_POWER) that the FP64 kernels use in place of the device
+ * library's, for each of n doubles of a device buffer, to check their accuracy (no counterpart in the
+ * reference).  Synchronises the device. */
+enum { PU_FN_ROOT = 0, PU_FN_POWER = 1 };
+int  pu_eval_fp64(int fn, const double *x, double a, double *y, long long n);
+
 /* Library build information (gfx target, precision variants compiled). */
 const char *pu_build_info(void);
 

@@ -94,6 +94,7 @@ def lib():
         "pu_memcpy_d2d": (I, [P, P, S]),
         "pu_measure_fma_rate": (I, [I, C.POINTER(D)]),
         "pu_measure_copy_rate": (I, [S, C.POINTER(D)]),
+        "pu_eval_fp64": (I, [I, P, D, P, C.c_longlong]),
         "pu_driver_create": (I, [I, I, I, I, D, I, I, C.c_ulonglong, I, C.c_char_p, C.POINTER(P)]),
         "pu_driver_step": (I, [P, I]),
         "pu_driver_set_forcing": (I, [P, P]),
@@ -437,6 +438,17 @@ class Dycore:
             self.destroy()
         except Exception:
             pass
+
+
+def eval_fp64(fn, x, a=0.):
+    """The FP64 kernels' square root ("root") or power x^a ("power") of each element, on the device."""
+    x = np.ascontiguousarray(x, dtype=np.float64)
+    d, y = DeviceBuffer(x.nbytes), DeviceBuffer(x.nbytes)
+    d.upload(x)
+    check(lib().pu_eval_fp64({"root": 0, "power": 1}[fn], d.ptr, a, y.ptr, x.size))
+    out = y.download(np.float64, x.shape)
+    d.free(); y.free()
+    return out
 
 
 def measure_ceilings(copy_bytes=2 << 30):

