@@ -288,12 +288,14 @@ __global__ __launch_bounds__(256) void k_sweep_zwall(const T *__restrict__ prim,
 // y sweep along periodic lines (adds to the tendencies), chunks of BS cells with an LDS carry.  The
 // periodic face between cells N-1 and 0 is computed last, by the thread of cell N-1, from cell 0's
 // lower values kept in LDS; the tendencies of cells 0 and N-1, which need it, are finished after the
-// last chunk.  At most 80 VGPRs (6 waves per SIMD; at 72 it spills and runs 1 % slower).
-#ifndef PU_YLINE_F32_WAVES
-#define PU_YLINE_F32_WAVES 6
-#endif
+// last chunk.
+//   Waves per SIMD by order: the low orders fit 72 VGPRs, and the schedule made for seven waves runs faster there
+// than the one for six; the high ones lose more to the spills that 72 cost them (us per launch at 7 and 6:
+// 700x24x144 order 3 122, 135, order 5 148, 163, order 7 168, 183, order 9 219, 210; 512x256x128 order 3
+// 664, 714, order 5 817, 879, order 7 944, 995).  With six order 9 still spills 1 VGPR and order 11 7.
+constexpr int yline_f32_waves(int ord) { return ord <= 7 ? 7 : 6; }
 template <int ORD, class T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PU_YLINE_F32_WAVES)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(yline_f32_waves(ORD))))
 void k_sweep_yline(const T *__restrict__ prim, const uint16_t *__restrict__ codes,
                                                              T *__restrict__ tend,
                                                      SweepParams P) {
