@@ -451,10 +451,14 @@ void k_sweep_yline(const T *__restrict__ prim, const uint16_t *__restrict__ code
 template <int DIR> struct SegShape { static constexpr int BX = 8, BY = 32, BS = 32; };
 template <> struct SegShape<0> { static constexpr int BX = 64, BY = 4, BS = 64; };
 
-// x: at most 80 VGPRs (6 waves per SIMD): 2.93 ms per launch at 512x512x128; 72 VGPRs run the same
-#ifndef PU_X_F32_WAVES
-#define PU_X_F32_WAVES 6
-#endif
+// x, waves per SIMD by order: up to WENO-5 the kernel fits 64 VGPRs; above that 80 leave room for loads in
+// flight (us per launch at 8 and 6 waves: 512x256x128 order 3 875, 939, order 5 1011, 1036, order 7 1200,
+// 1176, order 9 1521, 1418).
+constexpr int x_f32_waves(int ord) { return ord <= 5 ? 8 : 6; }
+// Whether a wave's row is worked out in scalar registers.  Orders 7 and 9 run 0.5 to 1 % slower so, order 3
+// 8 % and order 11 1 % faster (124x90x40 order 3 35.0 and 29.2 us with the wave cap; 512x256x128 order 11
+// 1949, 1928).
+constexpr bool x_f32_scalar_row(int ord) { return ord <= 5 || ord >= 11; }
 // a - b, never fused with the product that made one of them
 template <class T> __device__ __forceinline__ T plain_difference(T a, T b) {
 #pragma clang fp contract(off)
@@ -462,7 +466,7 @@ template <class T> __device__ __forceinline__ T plain_difference(T a, T b) {
 }
 
 template <int ORD, class T, int DIR, int MODE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIR == 0 ? PU_X_F32_WAVES : 1)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIR == 0 ? x_f32_waves(ORD) : 1)))
 void k_sweep(const T *__restrict__ prim, const uint16_t *__restrict__ codes,
                                                              T *__restrict__ tend,
                                                SweepParams P, FuseArgs<T> FA) {
@@ -474,7 +478,9 @@ void k_sweep(const T *__restrict__ prim, const uint16_t *__restrict__ codes,
   constexpr int NS = DIR == 0 ? 1 : NT;
   __shared__ T bufA0[NS], bufA1[NS], bufA2[NS], bufB0[NS], bufB1[NS];
 
-  const int tx = threadIdx.x, ty = threadIdx.y, lin = ty * BX + tx;
+  const int tx = threadIdx.x;
+  const int ty = DIR == 0 && x_f32_scalar_row(ORD) ? __builtin_amdgcn_readfirstlane(threadIdx.y) : (int)threadIdx.y;
+  const int lin = ty * BX + tx;
   const int t = DIR == 0 ? tx : ty;
   constexpr int nbs = DIR == 0 ? 1 : BX;
   unsigned bx, by, bz;
