@@ -94,30 +94,15 @@ def cpu_baseline(cfg_full, les, seconds_budget=25.0):
                       (cfg["name"].split("_1024")[0], cfg["nx"], cfg["ny"], cfg["nz"], steps, t_tot)}
 
 
-def by_segments(cfg, fam, fp64):
-    """The launch rule between whole lines and segments (by_segments of dycore_kernels.hip)."""
-    y, low = fam == "weno_y", cfg["ord"] < 9
-    if y and not fp64:
-        return False
-    rel = (0.77 if y else 0.9) if low else 0.96 if y else 1.03 if fp64 else 1.0
-    cells = cfg["ny"] if y else cfg["nz"]
-    blocks = -(-cfg["nx"] // 8) * (cfg["nz"] if y else cfg["ny"])
-    return rel * -(-cells // 30) < -(-cells // 32) * (1 + (320 if y else 240) / blocks)
-
-
 def sweep_kernel_name(cfg, fam):
-    """The kernel that runs sweep family `fam` (the launch choice of dycore_kernels.hip): z between
-    solid walls and periodic y lines the line kernels where by_segments does not choose otherwise, x
-    k_sweep_x in FP64 (which finishes the stage: MODE 2), otherwise the segment kernels (FP32 kernels
-    live in namespace f32)."""
+    """The kernel that runs sweep family `fam`: z and y the line kernels or the segment kernels, as
+    pu_sweep_route says; x k_sweep_x in FP64 (which finishes the stage: MODE 2) and the segment kernel
+    in FP32 (FP32 kernels live in namespace f32)."""
     import porturb_amd as pa
     fp64 = cfg["precision"] == pa.PU_FP64
     t, ns = ("double", "") if fp64 else ("float", "f32::")
-    lines = fam != "weno_x" and not by_segments(cfg, fam, fp64)
-    if lines and fam == "weno_z" and cfg["bc_z"] == pa.PU_BC_SOLID_WALL:
-        return "%sk_sweep_zwall<%d, %s>" % (ns, cfg["ord"], t)
-    if lines and fam == "weno_y" and cfg["bc_y"] == pa.PU_BC_PERIODIC and cfg["ny"] >= 2:
-        return "%sk_sweep_yline<%d, %s>" % (ns, cfg["ord"], t)
+    if fam != "weno_x" and not pa.sweep_takes_segments(cfg, 1 if fam == "weno_y" else 2):
+        return "%sk_sweep_%s<%d, %s>" % (ns, "yline" if fam == "weno_y" else "zwall", cfg["ord"], t)
     if fam == "weno_x" and fp64:
         return "k_sweep_x<%d, %s, 2>" % (cfg["ord"], t)
     d = {"weno_x": 0, "weno_y": 1, "weno_z": 2}[fam]

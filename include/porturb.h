@@ -282,6 +282,11 @@ enum { PU_CASE_BUBBLE = 1, PU_CASE_ABL_URBAN = 2, PU_CASE_WINDFARM = 3 };
 int  pu_case_init(const pu_config *cfg, int case_id, unsigned long long seed,
                   pu_coupler_state *cs, double *immersed_out);
 
+/* Which kernel the y (dir 1) or z (dir 2) sweep of a configuration takes: *segments 0 the whole-line kernel, 1
+ * the segment kernel (no counterpart in the reference; no device call; the environment variables that
+ * force a route when a context is created are not looked at). */
+int  pu_sweep_route(const pu_config *cfg, int dir, int *segments);
+
 /* Timing on the context's stream with HIP events.  pu_timer_* brackets a region;
  * pu_kernel_timing turns on per-launch events around the named kernel family ("weno_x",
  * "weno_y", "weno_z", "prep", "combine", "les") and pu_kernel_time reads the accumulated

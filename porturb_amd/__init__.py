@@ -85,6 +85,7 @@ def lib():
         "pu_synchronize": (I, [P]),
         "pu_case_init": (I, [cfgp, I, C.c_ulonglong, csp, P]),
         "pu_timer_start": (I, [P]),
+        "pu_sweep_route": (I, [C.POINTER(PuConfig), I, C.POINTER(I)]),
         "pu_timer_stop": (I, [P, C.POINTER(D)]),
         "pu_kernel_timing": (I, [P, I]),
         "pu_kernel_time": (I, [P, C.c_char_p, C.POINTER(D), C.POINTER(C.c_longlong)]),
@@ -438,6 +439,13 @@ class Dycore:
             self.destroy()
         except Exception:
             pass
+
+
+def sweep_takes_segments(cfg, direction):
+    """Whether the y (1) or z (2) sweep of a configuration runs by segments (else by whole lines)."""
+    out = C.c_int()
+    check(lib().pu_sweep_route(C.byref(to_pu_config(cfg)), direction, C.byref(out)))
+    return bool(out.value)
 
 
 def eval_fp64(fn, x, a=0.):

@@ -59,6 +59,17 @@ template <class P> static int alloc(P **p, size_t bytes) {
   return PU_OK;
 }
 
+static Grid grid_of(const pu_config &c) {
+  Grid g{};
+  g.nx = c.nx; g.ny = c.ny; g.nz = c.nz;
+  g.hs = (c.ord - 1) / 2;
+  g.hp = prim_halo(g.hs);
+  g.ox = PRIM_OX;
+  g.nxh = (g.ox + g.nx + g.hp + PRIM_ROW_ALIGN - 1) / PRIM_ROW_ALIGN * PRIM_ROW_ALIGN;
+  g.nyh = g.ny + 2 * g.hp; g.nzh = g.nz + 2 * g.hp;
+  return g;
+}
+
 static void free_ctx(pu_ctx *c) {
   void *ptrs[] = {c->d_hy, c->d_codes, c->d_any10, c->d_tau, c->d_relax, c->d_imm_les, c->d_imm_les_val,
                   c->d_U, c->d_Us, c->d_Ulo, c->d_Uslo, c->d_tend, c->d_prim, c->d_les, c->d_red,
@@ -93,16 +104,11 @@ int pu_create(const pu_config *cfg, void *stream, pu_ctx **out) {
   c->stream = (hipStream_t)stream;
   if (hipGetDevice(&c->device) != hipSuccess) { delete c; return fail(PU_ERR_HIP, "hipGetDevice failed"); }
   if (getenv("PORTURB_SEGMENT_SWEEPS")) {
-    const char *dirs = getenv("PORTURB_SEGMENT_DIRS");      // optional subset, e.g. "z" or "xy"
-    for (int d = 0; d < 3; d++) c->sweep_route[d] = !dirs || strchr(dirs, "xyz"[d]) ? pu_ctx::ROUTE_SEGMENTS : pu_ctx::ROUTE_LINES;
+    const char *dirs = getenv("PORTURB_SEGMENT_DIRS");      // optional subset: "y", "z", "yz" or nothing
+    for (int d = 1; d < 3; d++) c->sweep_route[d] = !dirs || strchr(dirs, "xyz"[d]) ? pu_ctx::ROUTE_SEGMENTS : pu_ctx::ROUTE_LINES;
   }
+  c->g = grid_of(*cfg);
   Grid &g = c->g;
-  g.nx = cfg->nx; g.ny = cfg->ny; g.nz = cfg->nz;
-  g.hs = (cfg->ord - 1) / 2;
-  g.hp = prim_halo(g.hs);
-  g.ox = PRIM_OX;
-  g.nxh = (g.ox + g.nx + g.hp + PRIM_ROW_ALIGN - 1) / PRIM_ROW_ALIGN * PRIM_ROW_ALIGN;
-  g.nyh = g.ny + 2 * g.hp; g.nzh = g.nz + 2 * g.hp;
   c->nv = NUM_STATE + cfg->num_tracers;
   c->nf = c->nv + 1;
   size_t n3 = (size_t)g.n3(), nh = (size_t)g.nh();
@@ -131,6 +137,15 @@ int pu_create(const pu_config *cfg, void *stream, pu_ctx **out) {
   hipEventCreate(&c->t0);
   hipEventCreate(&c->t1);
   *out = c;
+  return PU_OK;
+}
+
+int pu_sweep_route(const pu_config *cfg, int dir, int *segments) {
+  if (!segments) return fail(PU_ERR_ARG, "null output pointer");
+  int rc = validate(cfg);
+  if (rc) return rc;
+  if (dir != 1 && dir != 2) return fail(PU_ERR_ARG, "dir must be 1 (y) or 2 (z)");
+  *segments = rule_takes_segments(*cfg, grid_of(*cfg), dir) ? 1 : 0;
   return PU_OK;
 }
 

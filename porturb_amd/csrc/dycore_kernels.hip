@@ -346,28 +346,50 @@ static SweepParams sweep_params(pu_ctx *ctx, int dir) {
   return P;
 }
 
+// Whether the line kernel of a direction can run: z between solid walls, y periodic, lane offsets in 32 bits.
+static bool lines_apply(const pu_config &c, const Grid &g, int dir) {
+  const size_t es = c.precision == PU_FP32 ? sizeof(float) : sizeof(double);
+  return dir == 2 ? c.bc_z == PU_BC_SOLID_WALL && offsets_fit(g.nxh * g.nyh, g.hp, es)
+                  : c.bc_y == PU_BC_PERIODIC && offsets_fit(g.nxh, g.hp, es);
+}
+
 // Whole lines (blocks that walk CH_BX lines in chunks of CH_BS cells) or segments (blocks of SG_NC cells and
-// a neighbour at each end)?  A line's rounds are its chunks; the last round of blocks is part empty, which
-// costs about slots / blocks of a round; a segment's thread costs `rel` of a chunk's, less where the
-// order is low and the line's carries weigh more.  us per launch, lines then segments:
+// a neighbour at each end)?  A line's rounds are its chunks, in z with the last one at 0.6 and 0.1 for each
+// eight cells in it (waves without cells only wait); the last round of blocks is part empty, which costs about
+// slots / blocks of a round; a segment costs `rel` of a chunk.  The constants are fitted to both kernels' times
+// at 60 (FP32) and 40 (FP64) grids of 24 to 700 x 24 to 700 x 24 to 144 at each order; at 66 and 56 others
+// the kernel chosen in z took on average 1.001 to 1.006 of the faster one's time, at most 1.03 of the lines'.
+// us per launch, lines then segments:
 //   y FP64       512x512x128 order 5: 2715, 2108   order 9: 3679, 3925     500x310x90 order 5: 1242, 889
 //                96x200x33   order 9: 142, 83      64x64x64 order 5: 43, 30
 //   z FP64/FP32  512x512x128 order 5: 2268, 2573 / 1558, 1687   order 9: 3543, 4381 / 2342, 2834
 //                500x310x90  order 5: 959, 870 / 675, 593       order 9: 1494, 1477 / 1002, 976
 //                150x70x51   order 7: 74, 60 / 55, 51           16x16x128 order 9: 74, 23 / 70, 22
+//   z FP32       256x256x33  order 3: 147, 124  order 9: 213, 242  order 11: 296, 340
+//                300x200x100 order 3: 306, 245  order 9: 483, 501  order 11: 651, 703
+// Low orders in y: the one-sided reconstructions at the periodic end leave the FP64 line kernel 14 (order 5)
+// and 27 (order 7) spilled VGPRs, which its segments do not have.
 // In FP32 the y lines always take the line kernel: the two round differently there, and the limiter's map
 // would carry that into single cells (see sweep_f32_core.h).
-template <int ORD, class T> static bool by_segments(const pu_ctx *ctx, int dir, long long blocks, int cells) {
-  if (ctx->sweep_route[dir] != pu_ctx::ROUTE_RULE) return ctx->sweep_route[dir] == pu_ctx::ROUTE_SEGMENTS;
-  constexpr bool f32 = std::is_same<T, float>::value;
+bool rule_takes_segments(const pu_config &c, const Grid &g, int dir) {
+  if (!lines_apply(c, g, dir)) return true;
+  const bool f32 = c.precision == PU_FP32, low = c.ord < 9;
   if (f32 && dir == 1) return false;
-  const double rel = ORD < 9 ? (dir == 1 ? 0.77 : 0.9) : dir == 1 ? 0.96 : f32 ? 1. : 1.03;
+  const double rel = dir == 1 ? (low ? 0.77 : 0.96) : low ? 0.88 : f32 ? 0.98 : 1.;
   const double slots = dir == 1 ? 320. : 240.;
+  const double blocks = (double)((g.nx + CH_BX - 1) / CH_BX) * (dir == 1 ? g.nz : g.ny);
+  const int cells = dir == 1 ? g.ny : g.nz;
   const int chunks = (cells + CH_BS - 1) / CH_BS, segments = (cells + SG_NC - 1) / SG_NC;
-  return rel * segments < chunks * (1. + slots / (double)blocks);
+  const int rest = (cells - (chunks - 1) * CH_BS + 7) / 8;                    // eights of cells in the last chunk
+  const double line = dir == 1 ? chunks : chunks - 1 + 0.6 + 0.1 * rest;
+  return rel * segments < line * (1. + slots / blocks);
+}
+static bool takes_lines(const pu_ctx *ctx, int dir) {
+  if (ctx->sweep_route[dir] == pu_ctx::ROUTE_RULE) return !rule_takes_segments(ctx->cfg, ctx->g, dir);
+  return ctx->sweep_route[dir] == pu_ctx::ROUTE_LINES && lines_apply(ctx->cfg, ctx->g, dir);
 }
 
-// z sweep: writes d_tend.  Between solid walls by whole columns or segments (by_segments), otherwise
+// z sweep: writes d_tend.  Between solid walls by whole columns or segments (takes_lines), otherwise
 // (periodic z, or columns whose offsets need more than 32 bits) by segments.
 template <int ORD, class T>
 static int sweep_z(pu_ctx *ctx, hipStream_t s) {
@@ -378,7 +400,7 @@ static int sweep_z(pu_ctx *ctx, hipStream_t s) {
   T *tend = (T *)ctx->d_tend;
   const uint16_t *codes = ctx->d_codes + 2 * g.n3();
   const dim3 blk(CH_BX, CH_BS, 1), grd((unsigned)((g.nx + CH_BX - 1) / CH_BX), (unsigned)g.ny, 1);
-  if (P.wall_z && offsets_fit<T>(g.nxh * g.nyh, g.hp) && !by_segments<ORD, T>(ctx, 2, (long long)grd.x * grd.y, g.nz)) {
+  if (takes_lines(ctx, 2)) {
     if constexpr (std::is_same<T, float>::value) return launch_zwall_f32(ORD, grd, blk, s, prim, codes, tend, P);
     else hipLaunchKernelGGL((k_sweep_zwall<ORD, T>), grd, blk, 0, s, prim, codes, tend, P);
   } else if constexpr (std::is_same<T, float>::value) {
@@ -392,7 +414,7 @@ static int sweep_z(pu_ctx *ctx, hipStream_t s) {
   return PU_OK;
 }
 
-// y sweep: adds to d_tend.  Periodic lines by whole lines or segments (by_segments), otherwise segments.
+// y sweep: adds to d_tend.  Periodic lines by whole lines or segments (takes_lines), otherwise segments.
 template <int ORD, class T>
 static int sweep_y(pu_ctx *ctx, hipStream_t s) {
   const pu::Grid &g = ctx->g;
@@ -402,8 +424,7 @@ static int sweep_y(pu_ctx *ctx, hipStream_t s) {
   T *tend = (T *)ctx->d_tend;
   const uint16_t *codes = ctx->d_codes + g.n3();
   const dim3 blk(CH_BX, CH_BS, 1), grd((unsigned)((g.nx + CH_BX - 1) / CH_BX), (unsigned)g.nz, 1);
-  if (P.bc_along == PU_BC_PERIODIC && offsets_fit<T>(g.nxh, g.hp) &&
-      !by_segments<ORD, T>(ctx, 1, (long long)grd.x * grd.y, g.ny)) {
+  if (takes_lines(ctx, 1)) {
     if constexpr (std::is_same<T, float>::value) return launch_yline_f32(ORD, grd, blk, s, prim, codes, tend, P);
     else hipLaunchKernelGGL((k_sweep_yline<ORD, T>), grd, blk, 0, s, prim, codes, tend, P);
   } else if constexpr (std::is_same<T, float>::value) {

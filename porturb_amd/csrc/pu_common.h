@@ -52,10 +52,9 @@ struct pu_ctx {
   int nf = 0;                      // nv + 1           (reconstructed fields incl. pressure)
   bool dycore_ready = false;
   bool les_ready = false;
-  // sweeps through the segment kernel (environment variable PORTURB_SEGMENT_SWEEPS set when the
-  // context is created): the whole-line kernels are checked against it
-  // y and z sweeps: by the rule of by_segments, or (PORTURB_SEGMENT_SWEEPS) segments in the directions of
-  // PORTURB_SEGMENT_DIRS and whole lines in the others
+  // kernels of the y and z sweeps ([1], [2]): by the rule of rule_takes_segments or, where the environment variable
+  // PORTURB_SEGMENT_SWEEPS is set when the context is created, segments in the directions of
+  // PORTURB_SEGMENT_DIRS (both if that is not set) and whole lines where they apply in the others
   enum SweepRoute { ROUTE_RULE, ROUTE_LINES, ROUTE_SEGMENTS } sweep_route[3] = {ROUTE_RULE, ROUTE_RULE, ROUTE_RULE};
   // hydrostatic background, FP64 (host + device copies)
   std::vector<double> hy_cells[3];     // dens, theta, pressure: [nz+2hs]
@@ -234,6 +233,8 @@ int launch_c2d_prep(pu_ctx *ctx, const pu_coupler_state *cs, hipStream_t s);
 // stage combination (sources, SSPRK3 stage, clip, nrelax immersed relaxations) for every cell it
 // finishes
 int launch_sweeps(pu_ctx *ctx, hipStream_t s, int stage = -1, double dt = 0., int nrelax = 0);
+// whether the y (dir 1) or z (dir 2) sweep of a grid takes the segment kernel when no route is forced
+bool rule_takes_segments(const pu_config &c, const Grid &g, int dir);
 int launch_convert_c2d(pu_ctx *ctx, const pu_coupler_state *cs, int relax, hipStream_t s);
 int launch_convert_d2c(pu_ctx *ctx, pu_coupler_state *cs, hipStream_t s);
 int launch_tend_export(pu_ctx *ctx, double *tend, hipStream_t s);

@@ -329,9 +329,9 @@ __host__ __device__ constexpr int f64_waves(int ord) { return ord <= 9 ? 5 : 4; 
 constexpr int SW_NQ = 5 + PU_MAX_TRACERS;     // fluxes of a face: mass, normal momentum, transported
 
 // Whether the lane offsets of a line kernel (a chunk of 32 cells and its halo along the sweep) fit
-// 32 bits: sstride = elements between cells along the sweep.
-template <class T> static inline bool offsets_fit(long long sstride, int hp) {
-  return (CH_BS + 2 * hp + 2) * sstride * (long long)sizeof(T) + 4096 < (1LL << 32);
+// 32 bits: sstride = elements of es bytes between cells along the sweep.
+static inline bool offsets_fit(long long sstride, int hp, size_t es) {
+  return (CH_BS + 2 * hp + 2) * sstride * (long long)es + 4096 < (1LL << 32);
 }
 
 // ------------------------------------------------------------------------------------------------
