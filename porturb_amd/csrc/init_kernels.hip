@@ -74,8 +74,8 @@ __global__ __launch_bounds__(256) void k_hydro_means(const double *rd_, const do
 // Immersed precompute
 // ------------------------------------------------------------------------------------------------
 struct ImmParams {
-  int nx, ny, nz, hs, hp, ox;
-  long long nxh, nyh, nzh, n3;
+  int nx, ny, nz, hs;
+  long long n3;
   double power;
 };
 
@@ -88,43 +88,6 @@ __device__ __forceinline__ double imm_halo_value(const double *prop, int kh, int
   ih = ih < 0 ? 0 : (ih > nxh - 1 ? nxh - 1 : ih);
   if (kh < P.hs || kh >= P.hs + P.nz) return 1.;
   return prop[((long long)(kh - P.hs) * P.ny + wrapi_(jh - P.hs, P.ny)) * P.nx + wrapi_(ih - P.hs, P.nx)];
-}
-
-// flag array on the primitive halo (hp): prop > 0, z halos immersed
-__global__ __launch_bounds__(256) void k_imm_flag(const double *prop, uint8_t *flag, ImmParams P) {
-  long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  long long nh = P.nxh * P.nyh * P.nzh;
-  if (id >= nh) return;
-  int ih = (int)(id % P.nxh), jh = (int)((id / P.nxh) % P.nyh), kh = (int)(id / (P.nxh * P.nyh));
-  int k = kh - P.hp, j = jh - P.hp, i = ih - P.ox;
-  double v;
-  if (k < 0 || k >= P.nz) v = 1.;
-  else v = prop[((long long)k * P.ny + wrapi_(j, P.ny)) * P.nx + wrapi_(i, P.nx)];
-  flag[id] = v > 0 ? 1 : 0;
-}
-
-// Stencil codes of the sweeps along x, y and z (dynamics_rk.h:572-607 with
-// modify_stencil_immersed_der0, :478-493), fixed once the immersed cells are: how many points at
-// either end of a cell's stencil lie behind an immersed cell (0 for an immersed cell itself),
-// whether its two neighbours are immersed, and whether its 10-cell box holds an immersed cell.  The
-// sweeps read 2 bytes per cell instead of deriving them from 2 hs + 2 flag bytes in every launch.
-__global__ __launch_bounds__(256) void k_stencil_codes(const uint8_t *flag, const uint8_t *any10, uint16_t *codes,
-                                                       ImmParams P) {
-  const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (id >= P.n3) return;
-  const int i = (int)(id % P.nx), j = (int)((id / P.nx) % P.ny), k = (int)(id / ((long long)P.nx * P.ny));
-  const uint8_t *f = flag + ((long long)(k + P.hp) * P.nyh + (j + P.hp)) * P.nxh + (i + P.ox);
-  for (int d = 0; d < 3; d++) {
-    const long long st = d == 0 ? 1 : (d == 1 ? P.nxh : P.nxh * P.nyh);
-    int lo = 0, gap = 0;
-    if (!f[0]) {
-      for (int s = P.hs; s >= 1; s--) {          // the nearest immersed point decides
-        if (f[-s * st]) lo = P.hs - s + 1;
-        if (f[s * st]) gap = P.hs - s + 1;
-      }
-    }
-    codes[d * P.n3 + id] = (uint16_t)(lo | (gap << 4) | (f[-st] ? 0x100 : 0) | (f[st] ? 0x200 : 0) | (any10[id] ? 0x400 : 0));
-  }
 }
 
 // immersed tau (dynamics_rk.h:389-425) and relaxation multiplier pow(prop, power)/tau (:429)
@@ -166,19 +129,45 @@ __global__ __launch_bounds__(256) void k_any_y(const uint8_t *in, uint8_t *out, 
   for (int d = -R; d <= R; d++) m |= in[(k * P.ny + wrapi_(j + d, P.ny)) * P.nx + i];
   out[id] = m;
 }
-__global__ __launch_bounds__(256) void k_any_z(const uint8_t *in, uint8_t *out, ImmParams P, int R) {
-  long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (id >= P.n3) return;
-  long long plane = (long long)P.nx * P.ny;
-  int k = (int)(id / plane);
-  long long q = id - (long long)k * plane;
-  uint8_t m = 0;
-  for (int d = -R; d <= R; d++) {
-    int k2 = k + d;
-    if (k2 < 0 || k2 >= P.nz) continue;
-    m |= in[(long long)k2 * plane + q];
+// The z filter gives any_immersed10, and with it the stencil codes of the sweeps along x, y and z
+// (dynamics_rk.h:572-607 with modify_stencil_immersed_der0, :478-493), fixed once the immersed cells are: how
+// many points at either end of a cell's stencil lie behind an immersed cell (0 for an immersed cell
+// itself), whether its two neighbours are immersed, and whether its 10-cell box holds an immersed cell.
+// Levels beyond the domain count as immersed there (:1031-1034), x and y wrap.  The sweeps read 2 bytes per
+// cell instead of deriving them from 2 hs + 2 flags in every launch.  Only cells whose box holds an immersed
+// cell or which are near the walls look at their neighbours (pu_dycore_init at 300x200x100 920 us; 1020 with a
+// halo'd flag array and the codes in a pass of their own).  grid: (blocks over a level's nx*ny cells, nz levels).
+__global__ __launch_bounds__(256) void k_any_z_codes(const uint8_t *in, const double *prop, uint8_t *out, uint16_t *codes,
+                                                     ImmParams P, int R) {
+  const int plane = P.nx * P.ny, q = blockIdx.x * 256 + threadIdx.x, k = blockIdx.y;
+  if (q >= plane) return;
+  const long long id = (long long)k * plane + q;
+  uint8_t any = 0;
+  for (int c = max(k - R, 0); c <= min(k + R, P.nz - 1); c++) any |= in[(long long)c * plane + q];
+  out[id] = any;
+  if (!any && k >= P.hs && k < P.nz - P.hs) {          // the box covers the stencils but for the levels beyond
+    for (int d = 0; d < 3; d++) codes[d * P.n3 + id] = 0;
+    return;
   }
-  out[id] = m;
+  const int i = q % P.nx, j = q / P.nx;
+  auto wrap = [](int c, int n) { return c < 0 || c >= n ? wrapi_(c, n) : c; };
+  auto immersed = [&](int d, int s) {
+    const int kk = d == 2 ? k + s : k;
+    if (kk < 0 || kk >= P.nz) return true;
+    return prop[((long long)kk * P.ny + (d == 1 ? wrap(j + s, P.ny) : j)) * P.nx + (d == 0 ? wrap(i + s, P.nx) : i)] > 0;
+  };
+  const bool self = prop[id] > 0;
+  for (int d = 0; d < 3; d++) {
+    int lo = 0, gap = 0;
+    bool before = false, after = false;
+    for (int s = P.hs; s >= 1; s--) {                  // the nearest immersed point decides
+      before = immersed(d, -s);
+      after = immersed(d, s);
+      if (before && !self) lo = P.hs - s + 1;
+      if (after && !self) gap = P.hs - s + 1;
+    }
+    codes[d * P.n3 + id] = (uint16_t)(lo | (gap << 4) | (before ? 0x100 : 0) | (after ? 0x200 : 0) | (any ? 0x400 : 0));
+  }
 }
 
 // immersed_proportion_halos for the LES closure (sc_init.h:728-767): halo 1, x/y periodic,
@@ -302,8 +291,8 @@ static int upload_hydrostatics(pu_ctx *ctx) {
   return PU_OK;
 }
 
-// Immersed data from immersed_proportion: the flag array of the halo'd box
-// (dycore_immersed_proportion_halos > 0, dynamics_rk.h:1010-1030), tau and the relaxation
+// Immersed data from immersed_proportion: the stencil codes of
+// dycore_immersed_proportion_halos > 0 (dynamics_rk.h:1010-1030), tau and the relaxation
 // multiplier (:389-425), any_immersed10 (:1127-1143) and the closure's halo'd proportion
 // (sc_init.h:728-767).
 static int build_immersed(pu_ctx *ctx, const double *prop) {
@@ -312,20 +301,17 @@ static int build_immersed(pu_ctx *ctx, const double *prop) {
   hipStream_t s = ctx->stream;
   long long n3 = g.n3();
   ImmParams P;
-  P.nx = g.nx; P.ny = g.ny; P.nz = g.nz; P.hs = g.hs; P.hp = g.hp; P.ox = g.ox;
-  P.nxh = g.nxh; P.nyh = g.nyh; P.nzh = g.nzh; P.n3 = n3; P.power = c.immersed_power;
+  P.nx = g.nx; P.ny = g.ny; P.nz = g.nz; P.hs = g.hs; P.n3 = n3; P.power = c.immersed_power;
   dim3 grd((unsigned)((n3 + 255) / 256)), blk(256);
   hipLaunchKernelGGL(k_tau_relax, grd, blk, 0, s, prop, ctx->d_tau, ctx->d_relax, P);
   PU_HIP_CHECK(hipGetLastError());
-  const long long nh = g.nh();
-  uint8_t *tmp1 = nullptr, *tmp2 = nullptr;      // tmp1: a filter's result, then the halo'd flags
-  PU_HIP_CHECK(hipMalloc(&tmp1, nh));
+  uint8_t *tmp1 = nullptr, *tmp2 = nullptr;
+  PU_HIP_CHECK(hipMalloc(&tmp1, n3));
   PU_HIP_CHECK(hipMalloc(&tmp2, n3));
   hipLaunchKernelGGL(k_any_x, grd, blk, 0, s, prop, tmp1, P, 10);
   hipLaunchKernelGGL(k_any_y, grd, blk, 0, s, tmp1, tmp2, P, 10);
-  hipLaunchKernelGGL(k_any_z, grd, blk, 0, s, tmp2, ctx->d_any10, P, 10);
-  hipLaunchKernelGGL(k_imm_flag, dim3((unsigned)((nh + 255) / 256)), blk, 0, s, prop, tmp1, P);
-  hipLaunchKernelGGL(k_stencil_codes, grd, blk, 0, s, tmp1, ctx->d_any10, ctx->d_codes, P);
+  hipLaunchKernelGGL(k_any_z_codes, dim3((unsigned)((g.nx * g.ny + 255) / 256), (unsigned)g.nz), blk, 0, s, tmp2, prop,
+                     ctx->d_any10, ctx->d_codes, P, 10);
   PU_HIP_CHECK(hipGetLastError());
   long long nl = (long long)(g.nx + 2) * (g.ny + 2) * (g.nz + 2);
   hipLaunchKernelGGL(k_imm_les, dim3((unsigned)((nl + 255) / 256)), blk, 0, s, prop, ctx->d_imm_les_val,

@@ -54,7 +54,7 @@ template <class T, int S> __device__ __forceinline__ void excl_products(const T 
   for (int m = S - 1; m >= 0; m--) { P[m] = pre[m] * suf; suf *= D[m]; }
 }
 
-// Stencil code of a cell along one direction (k_stencil_codes, init_kernels.hip): 0 for a cell whose
+// Stencil code of a cell along one direction (k_any_z_codes, init_kernels.hip): 0 for a cell whose
 // stencil and 10-cell box hold no immersed cell.  In the order the stencil is read, `lo` points at
 // its start and `gap` points at its end are immersed ones to be replaced by the nearest valid point
 // (dynamics_rk.h:478-493), `first` / `last` tell whether the neighbour before / after the cell is
