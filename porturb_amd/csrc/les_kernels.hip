@@ -148,7 +148,8 @@ __device__ __forceinline__ Face<T> face_flux(const TileBox<T> &B, const LesParam
       tb = B.tau[DIR * B.n3 + gc];
     }
   };
-  // read ahead in FP32; in FP64 their registers would cost a wave of the four per SIMD
+  // read ahead in FP32; in FP64 that takes 133 VGPRs instead of 122, a wave less where LDS has room for four blocks,
+  // and where it has not (three diffused tracers, 500x310x60) ran 1037 us instead of 1032
   if (sizeof(T) == 4 && B.tau) load_tau();
   const T h = T(0.5);
   const T rdx = C.rdx, rdy = C.rdy, rdz = C.rdz, r2dx = C.r2dx, r2dy = C.r2dy, r2dz = C.r2dz;
@@ -257,11 +258,13 @@ struct FaceSlots {
 // (fields rho_d, u, v, w, theta, K and the diffused tracers, and the box points' immersed codes as
 // bytes) are staged in LDS once.  Each thread evaluates the three low faces of its cell; the tile's 144
 // high faces are a fourth face of waves 0 (y), 1 (z) and 2 (x).  The fluxes wait in the LDS of the box's
-// first fields, which nothing reads any more after the TKE source, so that four blocks fit a CU in FP64:
+// first fields, which nothing reads any more after the TKE source, so that they take no LDS of their own:
 // what bounds the kernel is the latency of its dependent chains (two square roots and two reciprocals a
-// face, about 40 LDS reads) at the waves that fit, and time falls with their number (with three blocks a
-// CU the same work took 1.4 times as long).  384x250x100 in FP64 with the prim kernel: 1030 us when
-// each cell computed its six faces, 918 us now; 512x256x128 in FP32 with learned stresses 1425 and 1316 us.
+// face, about 40 LDS reads) at the waves that fit.  In FP64 a block takes 31.8 KB and 5.2 KB for each
+// diffused tracer: four blocks a CU (as many as 122 VGPRs allow) with none or one, three with two or three
+// (the usual four tracers of which three diffuse); in FP32 half of that, six blocks (77 VGPRs) up to three.
+// With the prim kernel, us when each cell computed its six faces and now, three diffused tracers: 384x250x100
+// in FP64 960, 871; 512x256x128 in FP32 1182, 1140, with learned stresses 1419, 1296.
 // T = double: the reference's update in FP64 (les_closure.h:280-320, :404-413).  T = float: the
 // tendencies in FP32, applied as increments to the FP64 coupler entries (u += dt tend_u / rho,
 // T *= (1 + dt tend_theta / (rho theta))^gamma, TKE and tracer masses += dt tend), so the entries
@@ -526,7 +529,7 @@ template <class T>
 static int launch_les_update(pu_ctx *ctx, pu_coupler_state *cs, const LesParams &P, const TracerPtrs &tp) {
   const dim3 grd((unsigned)((P.nx + LTX - 1) / LTX), (unsigned)((P.ny + LTY - 1) / LTY), (unsigned)((P.nz + LTZ - 1) / LTZ));
   // box fields (<= 114 KB for 16 tracers in FP64), the immersed codes and the network's flags
-  const size_t lds = sizeof(T) * TileBox<T>::n * (6 + P.nq) +  TileBox<T>::n * (P.sflags ? 2 : 1);
+  const size_t lds = sizeof(T) * TileBox<T>::n * (6 + P.nq) + TileBox<T>::n * (P.sflags ? 2 : 1);
   if (lds > 65536)
     PU_HIP_CHECK(hipFuncSetAttribute((const void *)k_les_update<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   hipLaunchKernelGGL(k_les_update<T>, grd, dim3(LES_THREADS), lds, ctx->stream, (const T *)ctx->d_les,

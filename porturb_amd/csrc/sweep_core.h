@@ -10,10 +10,11 @@
 // whose upwind cell is the upper one reads that cell's stencil in reverse order and takes the same
 // right-face expressions, so a wave with both directions runs one code path.  With the full limiter
 // that is 7 of 10 fields (4 tracers) at 0.6 of the operations.
-//   The kernels are bound by VALU issue (67-70 % of the SIMD cycles; 2900 instructions per cell and
-// sweep of ten fields, 4350 before).  At 1024x1024x128 WENO-9, ms per launch: z 18.1 -> 14.1, y 19.4 ->
-// 14.8, x 22.7 -> 16.3; of it the upwind side 0.84, the register cap with constants left in the loops
-// 0.95, offsets and bases without 64-bit address arithmetic 0.96.
+//   The kernels are bound by VALU issue (67-70 % of the SIMD cycles where every stencil takes the limiter, with 2900
+// instructions per cell and sweep of ten fields, 4350 before; 52-59 % where two fifths are flat).  At
+// 1024x1024x128 WENO-9, ms per launch: z 18.1 -> 14.1, y 19.4 -> 14.8, x 22.7 -> 16.3; of it the upwind side
+// 0.84, the register cap with constants left in the loops 0.95, offsets and bases without 64-bit address
+// arithmetic 0.96.
 // FP32 has kernels of its own (sweep_f32_core.h).
 #pragma once
 #include "pu_common.h"
@@ -270,7 +271,7 @@ template <int ORD, class OFF> struct UpwindStencil {
 };
 
 // acoustic upwind state of one face (dynamics_rk.h:640-651): mass flux, pressure, upwind side.  The
-// multiply-adds are written out, here and in carried(): every kernel then rounds a face's fluxes
+// multiply-adds are written out, here and in carried(): every FP64 kernel then rounds a face's fluxes
 // the same way, whatever code surrounds them.
 template <class T> struct Upw {
   T ru, p;
@@ -290,7 +291,9 @@ __device__ __forceinline__ Upw<T> riemann(T rL, T uL, T pL, T rR, T uR, T pR, T 
 }
 
 // Flux of a transported value: rounded by itself, never fused into the divergence that follows, so
-// that a face's two cells see the same flux and every kernel computes the same tendencies.
+// that a face's two cells see the same flux.  The z kernels, which store the divergence, then give the same
+// tendencies to the last bit; the y kernels add it to what z left, a sum that the compiler fuses differently in
+// lines and segments (1e-13 of a tendency).
 template <class T> __device__ __forceinline__ T carried(T ru, T v) {
 #pragma clang fp contract(off)
   return ru * v;
@@ -323,8 +326,10 @@ template <int DIR, bool PEEL, class US, class F> __device__ __forceinline__ void
 // FP32 likewise).
 constexpr int CH_BX = 8, CH_BS = 32;
 
-// FP64 sweeps: at most 96 VGPRs (5 waves per SIMD), which they fit without spills up to WENO-9
-// (WENO-11 spills up to 30 there and takes 4 waves)
+// FP64 sweeps: at most 96 VGPRs (5 waves per SIMD), 128 at WENO-11 (4 waves; 96 cost it up to 30 spills).
+// Spilled VGPRs as built: y lines 14 at WENO-5 and 27 at WENO-7 (the one-sided reconstructions at the periodic
+// end), x with the stage combination 6 and z lines 2 at WENO-9, elsewhere none.  At WENO-9 and 1024x1024x128 x
+// writes 11.8 GB a launch for 9.7 GB of results (without spills 9.7); z 10.2 and y, which spills nothing, 10.1.
 __host__ __device__ constexpr int f64_waves(int ord) { return ord <= 9 ? 5 : 4; }
 constexpr int SW_NQ = 5 + PU_MAX_TRACERS;     // fluxes of a face: mass, normal momentum, transported
 

@@ -1,4 +1,4 @@
-// sweep_f32_core.h -- the FP32 sweep kernels: the segment sweep k_sweep, the whole-column z sweep
+// sweep_f32_core.h -- the FP32 sweep kernels: the x and segment sweep k_sweep, the whole-column z sweep
 // k_sweep_zwall and the whole-line y sweep k_sweep_yline.  Every field is reconstructed on both sides of
 // a cell from its stencil in memory order.  The upwind-side evaluation of the FP64 sweeps
 // (sweep_core.h), which reads half of the stencils in reverse, is not used in FP32: the limiter's map

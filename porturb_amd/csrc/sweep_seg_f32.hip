@@ -1,6 +1,6 @@
 // sweep_seg_f32.hip -- the FP32 segment sweeps (k_sweep<ORD, float, DIR, MODE>, sweep_f32_core.h) in a
-// translation unit of their own, built with -mllvm -disable-machine-licm (porturb_amd/build.py): the
-// x sweep then takes 70 VGPRs at WENO-9 without spills.
+// translation unit of their own, for parallel compilation; like all sweeps built with -mllvm
+// -disable-machine-licm (porturb_amd/build.py): the x sweep then takes 70 VGPRs at WENO-9 without spills.
 #include "sweep_f32_core.h"
 
 namespace pu {

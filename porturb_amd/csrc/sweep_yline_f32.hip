@@ -1,5 +1,6 @@
 // sweep_yline_f32.hip -- the FP32 whole-line y sweep (f32::k_sweep_yline<ORD, float>, sweep_f32_core.h) in a
-// translation unit of its own, built with -mllvm -disable-machine-licm (porturb_amd/build.py).
+// translation unit of its own, for parallel compilation; like all sweeps built with -mllvm
+// -disable-machine-licm (porturb_amd/build.py).
 #include "sweep_f32_core.h"
 
 namespace pu {

@@ -1,5 +1,6 @@
 // sweep_zwall_f32.hip -- the FP32 whole-column z sweep (f32::k_sweep_zwall<ORD, float>, sweep_f32_core.h) in
-// a translation unit of its own, built with -mllvm -disable-machine-licm (porturb_amd/build.py):
+// a translation unit of its own, for parallel compilation; like all sweeps built with -mllvm
+// -disable-machine-licm (porturb_amd/build.py):
 // without it the compiler hoists the limiter's constants out of the chunk loop into registers and
 // the kernel loses a wave per SIMD.
 #include "sweep_f32_core.h"
